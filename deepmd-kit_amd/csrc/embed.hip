@@ -25,13 +25,13 @@
 // registers): no LDS round trip between layers.  The sum over slots of the
 // forward contraction needs the slot on the K side: each 16-channel block of
 // G is re-laid with channels on lanes and slots on K (through a per-wavefront
-// LDS tile for F32/F64; by an identity MFMA, A = G, B = I, in the BF16
-// kernels), then R^T x G accumulates xyz.  In the backward, the sums run over
-// channels, which are already on K.
+// LDS tile for F32; by an identity MFMA, A = G, B = I, in the 16-bit kernels),
+// then R^T x G accumulates xyz.  In the backward, the sums run over channels,
+// which are already on K.
 //
-// Precision: F32 (v_mfma_f32_16x16x4_f32) and F64 (v_mfma_f64_16x16x4_f64)
-// run the policy kernels below; BF16 (FP32 accumulate, FP32 activations) has
-// its own kernels in namespace bf (LDS-resident weights, K = 32 MFMA).
+// Precision: F32 (v_mfma_f32_16x16x4_f32) runs the policy kernels below; BF16
+// / FP16 (FP32 accumulate, FP32 activations) have their own kernels in
+// namespace bf (LDS-resident weights, K = 32 MFMA); FP64 is in embed_f64.hip.
 #include <type_traits>
 
 #include "dpk_common.h"
@@ -39,10 +39,16 @@
 #include "embed_image.h"
 
 namespace dpk {
+
+// embed_f64.hip
+int embed_f64(bool fwd, void* out, const void* em, const void* gx, const int* atype,
+              const void* params, const int* net_of, const int* ch_out, int ntypes, int nnets,
+              int res2, int res3, int has_idt, const ActSpec& act, int d3, const int* sec_host,
+              int natoms, int nnei, const int* nlist, const double* pad, hipStream_t st);
+
 namespace {
 
 typedef __attribute__((ext_vector_type(4))) float v4f;
-typedef __attribute__((ext_vector_type(4))) double v4d;
 typedef __attribute__((ext_vector_type(4))) short v4s;
 
 // 16-bit storage (raw bits) of descriptor / gradient tensors exchanged with
@@ -70,8 +76,7 @@ __device__ __forceinline__ float fast_tanh(float x) {
 }
 
 // Register i of lane group g of a 16x16 MFMA accumulator holds row chan(g, i)
-// (checked on the device by a lane-layout probe): 4g + i for the FP32 and
-// BF16 instructions, g + 4i for v_mfma_f64_16x16x4f64.  Every activation
+// = 4g + i (checked on the device by a lane-layout probe).  Every activation
 // block uses the same mapping for its channel index, so a layer's output
 // registers are the next layer's B operand unchanged.
 struct PolF32 {
@@ -91,33 +96,6 @@ struct PolF32 {
     mma(c, a, b);
   }
   __device__ static __forceinline__ real tanh_(real x) { return fast_tanh(x); }
-};
-
-struct PolF64 {
-  using real = double;
-  using acc_t = v4d;
-  using wt = double;
-  static constexpr int kPrec = DPK_PREC_F64;
-  __device__ static __forceinline__ int chan(int g, int i) { return g + 4 * i; }
-  __device__ static __forceinline__ acc_t zero() { return v4d{0.0, 0.0, 0.0, 0.0}; }
-  __device__ static __forceinline__ void mma(acc_t& c, const real a[4], const real b[4]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[i], c, 0, 0, 0);
-  }
-  __device__ static __forceinline__ void mma_w(acc_t& c, const wt* aw, int g, const real b[4]) {
-    const real a[4] = {aw[g], aw[g + 4], aw[g + 8], aw[g + 12]};
-    mma(c, a, b);
-  }
-  // tanh = 1 - 2 / (e^{2x} + 1): the library exp and a Newton-refined
-  // reciprocal (within 1 ulp), absolute error ~2 ulp of 1 and no branches;
-  // the library tanh spends several times the instructions (its small-|x|
-  // branch keeps the relative error, which the sums of the net do not need).
-  // |x| > 20 is clamped (tanh is +-1 there in FP64; keeps e^{2x} finite for
-  // the reciprocal's Newton steps); a NaN passes through.
-  __device__ static __forceinline__ real tanh_(real x) {
-    const real xc = x > 20.0 ? 20.0 : (x < -20.0 ? -20.0 : x);
-    return 1.0 - 2.0 * rcp_nr(exp(2.0 * xc) + 1.0);
-  }
 };
 
 // Compile-time net shape: resnet mode of layers 2 and 3 (0: none, 2: y +=
@@ -165,9 +143,8 @@ struct Net {
   using real = typename Pol::real;
   using wt = typename Pol::wt;
   const real* p;   // packed real parameters of this net
-  const wt* w2;    // A-operand weights W2^T [P2][P1] (rows s2 apart)
-  const wt* w3;    // A-operand weights W3^T [P3][P2] (rows s3 apart)
-  int s2 = P1, s3 = P2;
+  const wt* w2;    // A-operand weights W2^T [P2][P1]
+  const wt* w3;    // A-operand weights W3^T [P3][P2]
 };
 
 template <class Pol, int P1, int P2, int P3>
@@ -179,45 +156,6 @@ __device__ __forceinline__ Net<Pol, P1, P2, P3> net_at(const void* params, int k
   n.w2 = n.p + L::w2t;
   n.w3 = n.p + L::w3t;
   return n;
-}
-
-// LDS-resident weights of the FP64 kernels (one net for the whole launch):
-// W2^T and W3^T with rows padded by one element, so that the 16 rows of an
-// A fragment (lanes c = 0..15, 16 per LDS pass) fall in distinct banks.
-// In FP64 W3^T alone (64 KB) exceeds L1: read from L2 every tile, the
-// weights bound the kernels by load latency.
-constexpr int kLwWaves = 8;  // atoms (wavefronts) per workgroup sharing the copy
-template <int P1, int P2, int P3>
-struct LdsW {
-  static constexpr int s2 = P1 + 1, s3 = P2 + 1;
-  static constexpr int w3 = P2 * s2;
-  static constexpr int elems = w3 + P3 * s3;
-  // backward: a wavefront's dE/dxyz rows [4][gs] (4 pad elements: the four
-  // rows of a read fall in distinct banks)
-  static constexpr int gs = P3 + 4;
-};
-
-template <class Pol, int P1, int P2, int P3>
-__device__ __forceinline__ void stage_weights(typename Pol::real* w, const void* params) {
-  using L = NetLayout<P1, P2, P3>;
-  using LW = LdsW<P1, P2, P3>;
-  using real = typename Pol::real;
-  const real* p = static_cast<const real*>(params);
-  for (int q = threadIdx.x; q < P2 * P1; q += blockDim.x)
-    w[(q / P1) * LW::s2 + q % P1] = p[L::w2t + q];
-  for (int q = threadIdx.x; q < P3 * P2; q += blockDim.x)
-    w[LW::w3 + (q / P2) * LW::s3 + q % P2] = p[L::w3t + q];
-  __syncthreads();
-}
-
-template <class Pol, int P1, int P2, int P3>
-__device__ __forceinline__ void use_lds_weights(Net<Pol, P1, P2, P3>& n,
-                                                const typename Pol::real* w) {
-  using LW = LdsW<P1, P2, P3>;
-  n.w2 = w;
-  n.w3 = w + LW::w3;
-  n.s2 = LW::s2;
-  n.s3 = LW::s3;
 }
 
 // Forward through the three layers for the lane's slot; optionally the
@@ -264,8 +202,8 @@ __device__ __forceinline__ void run_net(const Net<Pol, P1, P2, P3>& net, typenam
     const int row = 16 * m + c;
 #pragma unroll
     for (int k = 0; k < M1; ++k) {
-      Pol::mma_w(a, net.w2 + (size_t)row * net.s2 + 16 * k, g, y1[k]);
-      if (TANGENT) Pol::mma_w(da, net.w2 + (size_t)row * net.s2 + 16 * k, g, d1[k]);
+      Pol::mma_w(a, net.w2 + (size_t)row * P1 + 16 * k, g, y1[k]);
+      if (TANGENT) Pol::mma_w(da, net.w2 + (size_t)row * P1 + 16 * k, g, d1[k]);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -291,8 +229,8 @@ __device__ __forceinline__ void run_net(const Net<Pol, P1, P2, P3>& net, typenam
     const int row = 16 * m + c;
 #pragma unroll
     for (int k = 0; k < M2; ++k) {
-      Pol::mma_w(a, net.w3 + (size_t)row * net.s3 + 16 * k, g, y2[k]);
-      if (TANGENT) Pol::mma_w(da, net.w3 + (size_t)row * net.s3 + 16 * k, g, d2[k]);
+      Pol::mma_w(a, net.w3 + (size_t)row * P2 + 16 * k, g, y2[k]);
+      if (TANGENT) Pol::mma_w(da, net.w3 + (size_t)row * P2 + 16 * k, g, d2[k]);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -317,12 +255,9 @@ __device__ __forceinline__ void run_net(const Net<Pol, P1, P2, P3>& net, typenam
 }
 
 // --------------------------------------------------------------- forward --
-// LW: the launch uses one net, whose W2^T / W3^T the workgroup (kLwWaves
-// atoms) holds in LDS (dynamic shared memory); otherwise four atoms per
-// workgroup read the weights through the caches.
-template <class Pol, int P1, int P2, int P3, class C, bool GEN, bool LW>
-__global__ void __launch_bounds__(LW ? 64 * kLwWaves : 256)
-    __attribute__((amdgpu_waves_per_eu(Pol::kPrec == DPK_PREC_F64 && !C::IDT ? 2 : 1))) k_embed_fwd(
+// Four atoms per workgroup read the weights through the caches.
+template <class Pol, int P1, int P2, int P3, class C, bool GEN>
+__global__ void __launch_bounds__(256) k_embed_fwd(
     typename Pol::real* __restrict__ xyz, const typename Pol::real* __restrict__ em,
     const int* __restrict__ atype, const void* params,
     const int* __restrict__ net_of, const int* __restrict__ ch_out, BlockInfo bi, int d3,
@@ -330,10 +265,7 @@ __global__ void __launch_bounds__(LW ? 64 * kLwWaves : 256)
   using real = typename Pol::real;
   using acc_t = typename Pol::acc_t;
   constexpr int M3 = P3 / 16;
-  constexpr int NW = LW ? kLwWaves : 4;
-  extern __shared__ __align__(16) unsigned char wsm[];
-  real* lw = reinterpret_cast<real*>(wsm);
-  if constexpr (LW) stage_weights<Pol, P1, P2, P3>(lw, params);
+  constexpr int NW = 4;
   const int atom = blockIdx.x * NW + (threadIdx.x >> 6);
   if (atom >= natoms) return;
   const int lane = threadIdx.x & 63;
@@ -350,7 +282,6 @@ __global__ void __launch_bounds__(LW ? 64 * kLwWaves : 256)
   const bool real_centre = atype[atom] >= 0;
   for (int t = 0; t < bi.ntypes; ++t) {
     Net<Pol, P1, P2, P3> net = net_at<Pol, P1, P2, P3>(params, net_of[ti * bi.ntypes + t]);
-    if constexpr (LW) use_lds_weights(net, lw);
     const int b0 = bi.sec[t];
     int b1 = bi.sec[t + 1];
     if (bi.nlist != nullptr) {  // stop at the last real neighbour; padding tail from bi.pad
@@ -409,9 +340,8 @@ __global__ void __launch_bounds__(LW ? 64 * kLwWaves : 256)
 }
 
 // -------------------------------------------------------------- backward --
-template <class Pol, int P1, int P2, int P3, class C, bool GEN, bool LW>
-__global__ void __launch_bounds__(LW ? 64 * kLwWaves : 256)
-    __attribute__((amdgpu_waves_per_eu(Pol::kPrec == DPK_PREC_F64 && !C::IDT ? 2 : 1))) k_embed_bwd(
+template <class Pol, int P1, int P2, int P3, class C, bool GEN>
+__global__ void __launch_bounds__(256) k_embed_bwd(
     typename Pol::real* __restrict__ net_deriv, const typename Pol::real* __restrict__ em,
     const typename Pol::real* __restrict__ gxyz, const int* __restrict__ atype,
     const void* params, const int* __restrict__ net_of,
@@ -419,10 +349,7 @@ __global__ void __launch_bounds__(LW ? 64 * kLwWaves : 256)
   using real = typename Pol::real;
   using acc_t = typename Pol::acc_t;
   constexpr int M3 = P3 / 16;
-  constexpr int NW = LW ? kLwWaves : 4;
-  extern __shared__ __align__(16) unsigned char wsm[];
-  real* lw = reinterpret_cast<real*>(wsm);
-  if constexpr (LW) stage_weights<Pol, P1, P2, P3>(lw, params);
+  constexpr int NW = 4;
   const int atom = blockIdx.x * NW + (threadIdx.x >> 6);
   if (atom >= natoms) return;
   const int lane = threadIdx.x & 63;
@@ -431,36 +358,22 @@ __global__ void __launch_bounds__(LW ? 64 * kLwWaves : 256)
   ti = ti < 0 ? 0 : ti;
   const real* e = em + (size_t)atom * nnei * 4;
   real* nd = net_deriv + (size_t)atom * nnei * 4;
-  // A operand gx[c][16m + chan(g, i)] / nnei (rows c >= 4 are zero): in
-  // registers, or (LW) as the wavefront's four rows [c][128] in LDS, which
-  // frees the 64 registers the FP64 backward would otherwise spill
+  // A operand gx[c][16m + chan(g, i)] / nnei (rows c >= 4 are zero)
   const real inv = real(1) / real(nnei);
-  real gxa[LW ? 1 : M3][4];
-  constexpr int GS = LdsW<P1, P2, P3>::gs;
-  real* gxl = lw + LdsW<P1, P2, P3>::elems + (size_t)(threadIdx.x >> 6) * 4 * GS;
-  if constexpr (LW) {
-    for (int q = lane; q < 4 * P3; q += 64) {
-      const int tc = ch_out[q % P3];
-      gxl[(q / P3) * GS + q % P3] =
-          tc >= 0 ? gxyz[(size_t)atom * 4 * d3 + (q / P3) * d3 + tc] * inv : real(0);
-    }
-    wave_sync();
-  } else {
+  real gxa[M3][4];
 #pragma unroll
-    for (int m = 0; m < M3; ++m)
+  for (int m = 0; m < M3; ++m)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        real v = real(0);
-        if (c < 4) {
-          const int tc = ch_out[16 * m + Pol::chan(g, i)];
-          if (tc >= 0) v = gxyz[(size_t)atom * 4 * d3 + c * d3 + tc] * inv;
-        }
-        gxa[m][i] = v;
+    for (int i = 0; i < 4; ++i) {
+      real v = real(0);
+      if (c < 4) {
+        const int tc = ch_out[16 * m + Pol::chan(g, i)];
+        if (tc >= 0) v = gxyz[(size_t)atom * 4 * d3 + c * d3 + tc] * inv;
       }
-  }
+      gxa[m][i] = v;
+    }
   for (int t = 0; t < bi.ntypes; ++t) {
     Net<Pol, P1, P2, P3> net = net_at<Pol, P1, P2, P3>(params, net_of[ti * bi.ntypes + t]);
-    if constexpr (LW) use_lds_weights(net, lw);
     const int b0 = bi.sec[t];
     int b1 = bi.sec[t + 1];
     if (bi.nlist != nullptr) {  // padding slots after the last real neighbour: dE/d em = 0
@@ -479,43 +392,19 @@ __global__ void __launch_bounds__(LW ? 64 * kLwWaves : 256)
       acc_t dR = Pol::zero(), Mx = Pol::zero();
       run_net<Pol, P1, P2, P3, C, true, GEN>(net, s, g, c, bi.act,
                                      [&](int m, const real (&Gm)[4], const real (&dGm)[4]) {
-        if constexpr (LW) {
-          real ga[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            ga[i] = c < 4 ? gxl[c * GS + 16 * m + Pol::chan(g, i)] : real(0);
-          Pol::mma(dR, ga, Gm);
-          Pol::mma(Mx, ga, dGm);
-        } else {
-          Pol::mma(dR, gxa[m], Gm);   // dR[comp][slot c], comp = chan(g, i)
-          Pol::mma(Mx, gxa[m], dGm);  // sum_k gx[i][k] dG[slot][k]
-        }
+        Pol::mma(dR, gxa[m], Gm);   // dR[comp][slot c], comp = chan(g, i)
+        Pol::mma(Mx, gxa[m], dGm);  // sum_k gx[i][k] dG[slot][k]
       });
-      // components 0..3 of slot c: (lane c, register comp) for 4g+i
-      // layouts, (lane c + 16 comp, register 0) for g+4i
-      real dr4[4], mx4[4];
-      if constexpr (Pol::kPrec == DPK_PREC_F64) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          dr4[q] = __shfl(dR[0], c + 16 * q, 64);
-          mx4[q] = __shfl(Mx[0], c + 16 * q, 64);
-        }
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          dr4[q] = dR[q];
-          mx4[q] = Mx[q];
-        }
-      }
+      // components 0..3 of slot c: lane c, register comp
       if (g == 0 && slot < b1) {
         const real r0 = e[slot * 4], r1 = e[slot * 4 + 1], r2 = e[slot * 4 + 2],
                    r3 = e[slot * 4 + 3];
-        const real ds = r0 * mx4[0] + r1 * mx4[1] + r2 * mx4[2] + r3 * mx4[3];
+        const real ds = r0 * Mx[0] + r1 * Mx[1] + r2 * Mx[2] + r3 * Mx[3];
         real* o = nd + (size_t)slot * 4;
-        o[0] = dr4[0] + ds;
-        o[1] = dr4[1];
-        o[2] = dr4[2];
-        o[3] = dr4[3];
+        o[0] = dR[0] + ds;
+        o[1] = dR[1];
+        o[2] = dR[2];
+        o[3] = dR[3];
       }
     }
   }
@@ -1133,23 +1022,18 @@ __global__ void __launch_bounds__(256) k_desc_bwd(RT* __restrict__ gxyz,
   }
 }
 
-template <int P1, int P2, int P3, class Pol, class C, bool GEN, bool LW>
-int launch_embed_w(bool fwd, void* out, const void* em, const void* gx, const int* atype,
-                   const void* params, const int* net_of, const int* ch_out, const BlockInfo& bi,
-                   int d3, int natoms, int nnei, hipStream_t st) {
+template <int P1, int P2, int P3, class Pol, class C, bool GEN>
+int launch_embed(bool fwd, void* out, const void* em, const void* gx, const int* atype,
+                 const void* params, const int* net_of, const int* ch_out, const BlockInfo& bi,
+                 int d3, int natoms, int nnei, hipStream_t st) {
   using real = typename Pol::real;
-  constexpr int NW = LW ? kLwWaves : 4;
-  // LW: the weights, and for the backward each wavefront's dE/dxyz rows
-  const size_t lds =
-      LW ? sizeof(real) * (LdsW<P1, P2, P3>::elems + (fwd ? 0 : (size_t)NW * 4 * LdsW<P1, P2, P3>::gs))
-         : 0;
-  dim3 grid(cdiv(natoms, NW)), block(64 * NW);
+  dim3 grid(cdiv(natoms, 4)), block(256);
   if (fwd) {
-    hipLaunchKernelGGL((k_embed_fwd<Pol, P1, P2, P3, C, GEN, LW>), grid, block, lds, st,
+    hipLaunchKernelGGL((k_embed_fwd<Pol, P1, P2, P3, C, GEN>), grid, block, 0, st,
                        static_cast<real*>(out), static_cast<const real*>(em), atype, params,
                        net_of, ch_out, bi, d3, natoms, nnei);
   } else {
-    hipLaunchKernelGGL((k_embed_bwd<Pol, P1, P2, P3, C, GEN, LW>), grid, block, lds, st,
+    hipLaunchKernelGGL((k_embed_bwd<Pol, P1, P2, P3, C, GEN>), grid, block, 0, st,
                        static_cast<real*>(out), static_cast<const real*>(em),
                        static_cast<const real*>(gx), atype, params, net_of, ch_out, bi, d3,
                        natoms, nnei);
@@ -1158,36 +1042,19 @@ int launch_embed_w(bool fwd, void* out, const void* em, const void* gx, const in
   return DPK_OK;
 }
 
-// FP64 with a single net: weights in LDS (a workgroup of kLwWaves atoms);
-// FP32 weights (half the bytes) are served by L1 and keep four atoms per
-// workgroup.
-template <int P1, int P2, int P3, class Pol, class C, bool GEN>
-int launch_embed(bool fwd, void* out, const void* em, const void* gx, const int* atype,
-                 const void* params, const int* net_of, const int* ch_out, const BlockInfo& bi,
-                 int d3, int natoms, int nnei, int nnets, hipStream_t st) {
-  if constexpr (Pol::kPrec == DPK_PREC_F64) {
-    if (nnets == 1)
-      return launch_embed_w<P1, P2, P3, Pol, C, GEN, true>(fwd, out, em, gx, atype, params,
-                                                           net_of, ch_out, bi, d3, natoms,
-                                                           nnei, st);
-  }
-  return launch_embed_w<P1, P2, P3, Pol, C, GEN, false>(fwd, out, em, gx, atype, params, net_of,
-                                                        ch_out, bi, d3, natoms, nnei, st);
-}
-
 template <class Pol>
 int launch_embed_cfg(bool fwd, void* out, const void* em, const void* gx, const int* atype,
                      const void* params, const int* net_of, const int* ch_out,
                      const BlockInfo& bi, int res2, int res3, int has_idt, int d3, int natoms,
-                     int nnei, int nnets, hipStream_t st) {
+                     int nnei, hipStream_t st) {
 #define DPK_POL_LAUNCH(R2, R3, I)                                                            \
   return bi.act.id == DPK_ACT_TANH                                                           \
              ? launch_embed<32, 64, 128, Pol, Cfg<R2, R3, I>, false>(                        \
                    fwd, out, em, gx, atype, params, net_of, ch_out, bi, d3, natoms, nnei,     \
-                   nnets, st)                                                                \
+                   st)                                                                \
              : launch_embed<32, 64, 128, Pol, Cfg<R2, R3, I>, true>(                         \
                    fwd, out, em, gx, atype, params, net_of, ch_out, bi, d3, natoms, nnei,     \
-                   nnets, st)
+                   st)
   const int v = (res2 ? 4 : 0) + (res3 ? 2 : 0) + (has_idt ? 1 : 0);
   switch (v) {
     case 0: DPK_POL_LAUNCH(0, 0, false);
@@ -1206,8 +1073,8 @@ int embed_common(bool fwd, void* out, int prec, const void* em, const void* gx,
                  const int* atype, const void* params, const void* image, const int* net_of,
                  const int* ch_out, int ntypes, int nnets, int P1, int P2, int P3, int res2,
                  int res3, int has_idt, int act, double act_param, int d3,
-                 const int* sec_host, int natoms, int nnei, const int* nlist, const float* pad,
-                 dpk_stream_t stream) {
+                 const int* sec_host, int natoms, int nnei, const int* nlist, const void* pad,
+                 dpk_stream_t stream, bool skip64 = false) {
   clear_error();
   DPK_REQUIRE(natoms >= 0 && nnei > 0, DPK_ERR_ARG, "embed: bad sizes");
   DPK_REQUIRE(ntypes > 0 && ntypes <= kMaxTypes, DPK_ERR_ARG, "embed: ntypes=%d", ntypes);
@@ -1228,7 +1095,7 @@ int embed_common(bool fwd, void* out, int prec, const void* em, const void* gx,
               act);
   bi.ntypes = ntypes;
   bi.nlist = prec != DPK_PREC_F64 ? nlist : nullptr;
-  bi.pad = prec != DPK_PREC_F64 ? pad : nullptr;
+  bi.pad = prec != DPK_PREC_F64 ? static_cast<const float*>(pad) : nullptr;
   for (int t = 0; t <= ntypes; ++t) bi.sec[t] = sec_host[t];
   DPK_REQUIRE(bi.sec[ntypes] == nnei, DPK_ERR_ARG, "embed: sum(sel)=%d != nnei=%d", bi.sec[ntypes], nnei);
   if (natoms == 0) return DPK_OK;
@@ -1258,10 +1125,11 @@ int embed_common(bool fwd, void* out, int prec, const void* em, const void* gx,
     }
     case DPK_PREC_F32:
       return launch_embed_cfg<PolF32>(fwd, out, em, gx, atype, params, net_of, ch_out, bi, res2,
-                                      res3, has_idt, d3, natoms, nnei, nnets, st);
+                                      res3, has_idt, d3, natoms, nnei, st);
     case DPK_PREC_F64:
-      return launch_embed_cfg<PolF64>(fwd, out, em, gx, atype, params, net_of, ch_out, bi, res2,
-                                      res3, has_idt, d3, natoms, nnei, nnets, st);
+      return embed_f64(fwd, out, em, gx, atype, params, net_of, ch_out, ntypes, nnets, res2, res3,
+                       has_idt, bi.act, d3, sec_host, natoms, nnei, skip64 ? nlist : nullptr,
+                       skip64 ? static_cast<const double*>(pad) : nullptr, st);
   }
   set_error("embed: unknown precision %d", prec);
   return DPK_ERR_ARG;
@@ -1325,6 +1193,28 @@ extern "C" int dpk_embed_bwd(void* net_deriv, int prec, const void* em, const vo
   return embed_common(false, net_deriv, prec, em, gxyz, atype, params, image, net_of, ch_out,
                       ntypes, nnets, P1, P2, P3, res2, res3, has_idt, act, act_param, d3, sec_host,
                       natoms, nnei, nlist, nullptr, stream);
+}
+
+extern "C" int dpk_embed_skip_fwd_f64(double* xyz, const double* em, const int* atype,
+                                      const double* params, const int* net_of, const int* ch_out,
+                                      int ntypes, int nnets, int P1, int P2, int P3, int res2,
+                                      int res3, int has_idt, int act, double act_param, int d3,
+                                      const int* sec_host, int natoms, int nnei, const int* nlist,
+                                      const double* pad, dpk_stream_t stream) {
+  return embed_common(true, xyz, DPK_PREC_F64, em, nullptr, atype, params, nullptr, net_of, ch_out,
+                      ntypes, nnets, P1, P2, P3, res2, res3, has_idt, act, act_param, d3, sec_host,
+                      natoms, nnei, nlist, pad, stream, true);
+}
+
+extern "C" int dpk_embed_skip_bwd_f64(double* net_deriv, const double* em, const double* gxyz,
+                                      const int* atype, const double* params, const int* net_of,
+                                      const int* ch_out, int ntypes, int nnets, int P1, int P2,
+                                      int P3, int res2, int res3, int has_idt, int act,
+                                      double act_param, int d3, const int* sec_host, int natoms,
+                                      int nnei, const int* nlist, dpk_stream_t stream) {
+  return embed_common(false, net_deriv, DPK_PREC_F64, em, gxyz, atype, params, nullptr, net_of,
+                      ch_out, ntypes, nnets, P1, P2, P3, res2, res3, has_idt, act, act_param, d3,
+                      sec_host, natoms, nnei, nlist, nullptr, stream, true);
 }
 
 template <typename RT, typename OT>

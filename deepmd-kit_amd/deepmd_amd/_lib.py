@@ -97,6 +97,12 @@ _SIGS = {
     "dpk_embed_bwd": (c_int, [P, c_int, P, P, P, P, P, P, P, c_int, c_int, c_int, c_int,
                               c_int, c_int, c_int, c_int, c_int, c_double, c_int, P, c_int,
                               c_int, P, P]),
+    "dpk_embed_skip_fwd_f64": (c_int, [P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int, c_int,
+                                       c_int, c_int, c_int, c_double, c_int, P, c_int, c_int, P,
+                                       P, P]),
+    "dpk_embed_skip_bwd_f64": (c_int, [P, P, P, P, P, P, P, c_int, c_int, c_int, c_int, c_int,
+                                       c_int, c_int, c_int, c_int, c_double, c_int, P, c_int,
+                                       c_int, P, P]),
     "dpk_embed_train_bimage_bytes": (c_size_t, []),
     "dpk_embed_train_pack_bwd": (c_int, [P, P, c_int, P]),
     "dpk_embed_train_parts_elems": (c_size_t, [c_int, c_int]),

@@ -312,7 +312,7 @@ def padding_table(packed, net_of, davg, dstd, sec, r2, r3, act="tanh"):
             G = embed_internal(packed[net_of[ti, t]], R[ti, a:b, 0], r2, r3, act)  # [b-a, 128]
             C = R[ti, a:b, :, None] * G[:, None, :]
             pad[ti, a:b] = np.cumsum(C[::-1], axis=0)[::-1]
-    return pad.astype(np.float32)
+    return pad
 
 
 # ---------------------------------------------------------------- fitting --
@@ -677,8 +677,8 @@ class SeAModel:
     Launch tunables (kernel organisations chosen by deepmd_amd.autotune) are
     the model's own (``self.tuning``), current around its launches."""
 
-    # 16-bit / FP32 embedding: compute each type block only up to its last real
-    # neighbour (padding rows from a table), dpk_embed_fwd / _bwd with nlist
+    # compute each type block only up to its last real neighbour (padding rows
+    # from a table): dpk_embed_fwd / _bwd with nlist, dpk_embed_skip_*_f64
     SKIP_PADDING = True
 
     def __init__(self, model_dict: dict, precision: str = "f64", device="cuda",
@@ -798,16 +798,16 @@ class SeAModel:
             for tb in range(nt):
                 net_of[ti, tb] = tb if self.type_one_side else tb * nt + ti
         self.net_of = torch.tensor(net_of.ravel(), dtype=torch.int32, device=dev)
-        # 16-bit / FP32: type blocks end at their last real neighbour, the
-        # padding tail comes from a per-(centre type, slot) table
+        # type blocks end at their last real neighbour, the padding tail comes
+        # from a per-(centre type, slot) table
         self.emb_pad = None
-        self.skip_padding = self.precision in HALF + ("f32",) and self.SKIP_PADDING
+        self.skip_padding = self.SKIP_PADDING
         if self.skip_padding:
             pad = padding_table(packed, net_of, self.davg.reshape(nt, self.nnei, 4),
                                 self.dstd.reshape(nt, self.nnei, 4), self.sec, r2, r3,
                                 self.emb_act_name)
             if pad is not None:
-                self.emb_pad = torch.from_numpy(pad).to(dev).contiguous()
+                self.emb_pad = torch.tensor(pad, dtype=real, device=dev).contiguous()
         self.pair_mask = None  # (ntypes+1)^2 type-pair table, exclude_mask.py:64-140
         if self.exclude_types:
             tab = np.ones((nt + 1, nt + 1), dtype=np.int32)
@@ -1278,6 +1278,11 @@ class SeAModel:
         (pp, pw, no, co, nt, nn, p1, p2, p3, r2, r3, hi, ac, ap, d3) = self._embed_args()
         nl = ptr(s.nlist) if self._skip_padding() else None
         pad = ptr(self.emb_pad) if nl is not None and self.emb_pad is not None else None
+        if self.precision == "f64":
+            call("dpk_embed_skip_fwd_f64", ptr(s.xyz), ptr(s.em), ptr(s.atype), pp, no, co, nt, nn,
+                 p1, p2, p3, r2, r3, hi, ac, ap, d3, self.sec_host[1], fs.natoms, self.nnei, nl,
+                 pad, st)
+            return
         call("dpk_embed_fwd", ptr(s.xyz), self.prec, ptr(s.em), ptr(s.atype), pp, pw, no, co,
              nt, nn, p1, p2, p3, r2, r3, hi, ac, ap, d3, self.sec_host[1], fs.natoms, self.nnei,
              nl, pad, st)
@@ -1294,6 +1299,11 @@ class SeAModel:
             return
         (pp, pw, no, co, nt, nn, p1, p2, p3, r2, r3, hi, ac, ap, d3) = self._embed_args()
         nl = ptr(s.nlist) if self._skip_padding() else None
+        if self.precision == "f64":
+            call("dpk_embed_skip_bwd_f64", ptr(s.nd), ptr(s.em), ptr(s.gxyz), ptr(s.atype), pp, no,
+                 co, nt, nn, p1, p2, p3, r2, r3, hi, ac, ap, d3, self.sec_host[1], fs.natoms,
+                 self.nnei, nl, st)
+            return
         call("dpk_embed_bwd", ptr(s.nd), self.prec, ptr(s.em), ptr(s.gxyz), ptr(s.atype), pp, pw,
              no, co, nt, nn, p1, p2, p3, r2, r3, hi, ac, ap, d3, self.sec_host[1], fs.natoms,
              self.nnei, nl, st)

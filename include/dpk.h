@@ -424,6 +424,31 @@ int dpk_embed_bwd(void* net_deriv, int prec, const void* em, const void* gxyz,
                   int natoms, int nnei, const int* nlist, dpk_stream_t stream);
 
 /*
+ * The FP64 forward and backward with padding left out, as nlist does for the
+ * other precisions of dpk_embed_fwd / _bwd (which compute every slot in FP64):
+ * each type block ends at its last real neighbour; pad is the FP64 form of
+ * that table, [ntypes, nnei, 4, 128] (NULL when every padding row is zero).
+ * The backward gives the padding slots their derivative all the same.
+ * nlist = NULL: every slot.
+ */
+int dpk_embed_skip_fwd_f64(double* xyz, const double* em, const int* atype,
+                           const double* params, const int* net_of,
+                           const int* ch_out, int ntypes, int nnets, int P1,
+                           int P2, int P3, int res2, int res3, int has_idt,
+                           int act, double act_param, int d3,
+                           const int* sec_host, int natoms, int nnei,
+                           const int* nlist, const double* pad,
+                           dpk_stream_t stream);
+int dpk_embed_skip_bwd_f64(double* net_deriv, const double* em,
+                           const double* gxyz, const int* atype,
+                           const double* params, const int* net_of,
+                           const int* ch_out, int ntypes, int nnets, int P1,
+                           int P2, int P3, int res2, int res3, int has_idt,
+                           int act, double act_param, int d3,
+                           const int* sec_host, int natoms, int nnei,
+                           const int* nlist, dpk_stream_t stream);
+
+/*
  * Training: the backward passes of the two embedding functions a force-loss
  * training step differentiates (replacing torch's double backward through
  * DescrptBlockSeA.forward, deepmd/pt/model/descriptor/se_a.py:784-858, with
