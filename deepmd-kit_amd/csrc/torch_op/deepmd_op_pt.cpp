@@ -143,8 +143,9 @@ std::vector<Tensor> tab_grad(const Tensor& table, const Tensor& info, const Tens
               dy.numel(), " values, expected ", a.nloc, " x ", a.nd, " x ", L);
   require_gpu(table, "tabulate_fusion_se_a_grad");
   const c10::DeviceGuard guard(table.device());
-  Tensor dx = torch::zeros_like(a.em_x);
-  Tensor dem = torch::zeros_like(a.em);
+  // (the kernels write every value)
+  Tensor dx = torch::empty_like(a.em_x);
+  Tensor dem = torch::empty_like(a.em);
   if (a.nloc == 0) return {dx, dem};
   Tensor dyc = dy.contiguous();
   void* st = stream_of(table);
