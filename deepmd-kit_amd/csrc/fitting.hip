@@ -475,6 +475,56 @@ __global__ void __launch_bounds__(256) k_desc_bwd_r(float* __restrict__ gxyz,
   }
 }
 
+// k_desc_bwd in FP64 for M2 = 16: one wavefront per slot, dE/dD straight from
+// memory (twice: the lane's own rows p for the first term, rows in turn for
+// the second, whose lanes are (m, k mod 4)), only xyz in LDS.  Staged rows of
+// 16 doubles put all lanes of the first term on one LDS bank: 72 us at 5,324
+// atoms (87 MB of dE/dD), 30 without.
+__global__ void __launch_bounds__(256) k_desc_bwd64(double* __restrict__ gxyz,
+                                                    const double* __restrict__ gd,
+                                                    const double* __restrict__ xyz,
+                                                    const int* __restrict__ order, int nslots,
+                                                    int d3) {
+  constexpr int M2 = 16;
+  __shared__ __align__(16) double xs[4][4 * kMaxD3];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int slot = blockIdx.x * 4 + wave;
+  if (slot >= nslots) return;  // no workgroup barrier below
+  const int atom = __builtin_amdgcn_readfirstlane(order[slot]);
+  double* x = xs[wave];
+  for (int q = lane; q < 4 * d3; q += 64) x[q] = xyz[(size_t)atom * 4 * d3 + q];
+  wave_sync_lds();
+  const double* g = gd + (size_t)slot * d3 * M2;
+  double b[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int k = lane >> 4; k < d3; k += 4) {
+    const double v = g[k * M2 + (lane & 15)];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) b[c] += v * x[c * d3 + k];
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    b[c] += __shfl_xor(b[c], 16, 64);
+    b[c] += __shfl_xor(b[c], 32, 64);
+  }
+  double* o = gxyz + (size_t)atom * 4 * d3;
+  for (int p = lane; p < d3; p += 64) {
+    double v[M2];
+#pragma unroll
+    for (int m = 0; m < M2; m += 2) {
+      const double2 u = *reinterpret_cast<const double2*>(g + (size_t)p * M2 + m);
+      v[m] = u.x;
+      v[m + 1] = u.y;
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      double a = p < M2 ? b[c] : 0.0;
+#pragma unroll
+      for (int m = 0; m < M2; ++m) a += v[m] * x[c * d3 + m];
+      o[c * d3 + p] = a;
+    }
+  }
+}
+
 // Descriptor rows without LDS staging: one wavefront per slot, lanes over
 // channels p (stride 64).  xyz[c][m] for m < M2 is wave-uniform (scalar
 // loads); the lane's own xyz[c][p] and its D row piece D[p][0..M2) stay in
@@ -649,6 +699,13 @@ extern "C" int dpk_fit_descriptor_bwd(void* gxyz, int prec, const void* gdesc, c
   DPK_REQUIRE(prec != DPK_PREC_F64 || lds_f64 <= 65536, DPK_ERR_UNSUPPORTED,
               "fit_descriptor_bwd: d3=%d m2=%d needs %zu B of LDS in FP64", d3, m2, lds_f64);
   if (prec == DPK_PREC_F16X2) prec = DPK_PREC_F32;  // split mode: dE/dD is FP32
+  if (m2 == 16 && prec == DPK_PREC_F64 && reinterpret_cast<size_t>(gdesc) % 16 == 0) {
+    hipLaunchKernelGGL(fit::k_desc_bwd64, dim3(cdiv(nslots, 4)), dim3(256), 0, st,
+                       static_cast<double*>(gxyz), static_cast<const double*>(gdesc),
+                       static_cast<const double*>(xyz), order, nslots, d3);
+    DPK_LAUNCHED();
+    return DPK_OK;
+  }
   if (m2 == 16 && prec != DPK_PREC_F64) {
     const int np = (d3 + 63) / 64;
 #define DPK_DESC_BWD_R(T, NP)                                                                    \

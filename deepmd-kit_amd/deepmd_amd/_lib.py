@@ -120,6 +120,9 @@ _SIGS = {
                                   c_double, P]),
     "dpk_fit_energy": (c_int, [P, P, c_int, P, P, P, c_double, P, c_int, c_int, P]),
     "dpk_fit_layer_bwd": (c_int, [P, P, c_int, P, P, P, P, c_int, c_int, c_int, c_int, P]),
+    "dpk_fit_chain_f64_workspace_bytes": (c_size_t, [c_int, c_int, P]),
+    "dpk_fit_chain_f64": (c_int, [c_int, P, P, P, P, c_int, P, P, P, P, P, c_int, c_int, c_int, P,
+                                  P, c_size_t, P]),
     "dpk_fit_tail_bytes": (c_size_t, [c_int]),
     "dpk_fit_tail_bf16": (c_int, [P, P, P, P, c_int, c_int, c_double, P, c_int, P]),
     "dpk_fit_tail_f16": (c_int, [P, P, P, P, c_int, c_int, c_double, P, c_int, P]),

@@ -327,7 +327,9 @@ class Fitting:
     product and the descriptor in/out in dpk_fit_energy /
     dpk_fit_descriptor_fwd / _bwd.  Hidden layers: tanh, optional idt, resnet
     0 / 1 / 2; output layer: linear to one value (the reference's
-    EnergyFittingNet, network.py:935-1006).  16-bit (BF16 / FP16) nets of 2
+    EnergyFittingNet, network.py:935-1006).  FP64 tanh nets of widths
+    divisible by 16 run as a whole in one call (dpk_fit_chain_f64).  16-bit (BF16 /
+    FP16) nets of 2
     or 3 hidden layers of (padded) width 256 run layers 2..L, the energy and
     the backward down to dE/dz_1 in one kernel (dpk_fit_tail_bf16 / _f16)
     between the layer-1
@@ -344,6 +346,8 @@ class Fitting:
     # split FP16: descriptor + layer 1 (and their backward) in one kernel each
     # (dpk_fit_l1_fwd / _bwd) instead of writing D and dE/dD around two GEMMs
     FUSED_L1 = True
+    # FP64 tanh nets: the whole fitting in one call (dpk_fit_chain_f64)
+    CHAIN = True
 
     def __init__(self, nets, bias_atom_e, out_bias, prec: str, device, nx: int = 0):
         self.prec = prec
@@ -440,6 +444,7 @@ class Fitting:
             self.tail_res = [sum(1 << (t - 1) for t in range(1, L) if net["hidden"][t]["res"] == 1)
                              for net in self.nets]
             assert all(t.numel() == lib().dpk_fit_tail_bytes(L) for t in self.tail)
+        self.chain = self._chain_plan() if self.CHAIN else None
         self.l1 = None
         if self.split and self.FUSED_L1 and self.din % 16 == 0:
             d3 = self.din // 16
@@ -452,6 +457,31 @@ class Fitting:
                     call("dpk_fit_l1_pack", ptr(img), DPK_PREC_F16X2, ptr(w1), d3, 16,
                          self.widths[0], stream_ptr())
                     self.l1.append(img)
+
+    def _chain_plan(self):
+        """Host tables of dpk_fit_chain_f64 (weights in its fragment order), or
+        None where it does not take these nets."""
+        if (self.prec != "f64" or self.act != ACTIVATIONS["tanh"] or self.nx
+                or len(self.nets) > 16 or len(self.widths) > 8
+                or any(w % 16 for w in [self.din] + self.widths)):
+            return None
+        L = len(self.widths)
+        keep, params, res = [], [], []
+
+        def address(t):
+            keep.append(t)
+            return 0 if t is None else t.data_ptr()
+
+        for net in self.nets:
+            for ly in net["hidden"]:
+                params += [address(pack_fit_chain(ly["w"])), address(pack_fit_chain(ly["wt"])),
+                           address(ly["b"]), address(ly["idt"])]
+                res.append(ly["res"])
+            params.append(address(net["wout"]))
+        ebias = [net["bout"] + float(b) for net, b in zip(self.nets, self.ebias)]
+        return dict(keep=keep, L=L, widths=ctypes_int_array([self.din] + self.widths),
+                    res=ctypes_int_array(res), params=ctypes_array(params, "longlong"),
+                    ebias=ctypes_array(ebias, "double"))
 
     @staticmethod
     def tail_shape(fit_layers) -> bool:
@@ -474,6 +504,10 @@ class Fitting:
                     "D": torch.empty((nd, 2 * self.din), dtype=gd, device=dev),
                     "GD": torch.empty((nd, self.din), dtype=torch.float32, device=dev),
                     "cx": None}
+        if self.chain is not None:
+            nb = int(lib().dpk_fit_chain_f64_workspace_bytes(n, nl, self.chain["widths"][1]))
+            return {"D": torch.empty((n, self.din), dtype=gd, device=dev),
+                    "ws": torch.empty(max(nb, 1), dtype=torch.uint8, device=dev)}
         bf = {
             "z": torch.empty(n * hmax, dtype=gd, device=dev),
             "y": [torch.empty(n * hmax, dtype=rd, device=dev) for _ in range(2)],
@@ -512,6 +546,13 @@ class Fitting:
         pc = self.prec_code
         if self.nx and xe is None:
             raise ValueError("the fitting nets take frame / atomic parameters: xe is required")
+        if self.chain is not None:
+            ch = self.chain
+            segs = ctypes_int_array([v for seg in segments for v in seg])
+            call("dpk_fit_chain_f64", ch["L"], ch["widths"][1], ch["res"][1], ch["params"][1],
+                 ch["ebias"][1], len(segments), segs[1], ptr(atom_e), ptr(gxyz), ptr(xyz),
+                 ptr(order), n, d3, m2, ptr(bf["D"]), ptr(bf["ws"]), bf["ws"].numel(), st)
+            return
         fused = self.l1 is not None and m2 == 16 and d3 * 16 == self.din
         if not fused:
             call("dpk_fit_descriptor_fwd", ptr(bf["D"]), pc, ptr(xyz), ptr(order), n, d3, m2, st)
@@ -604,6 +645,13 @@ def _tail_fragment_index():
     row = np.broadcast_to(16 * mb + m, (16, 8, 4, 16, 8)).reshape(-1)
     col = np.broadcast_to(32 * kc + 16 * (j // 4) + 4 * g + j % 4, (16, 8, 4, 16, 8)).reshape(-1)
     return row, col
+
+
+def pack_fit_chain(w: torch.Tensor) -> torch.Tensor:
+    """A weight [K, N] (multiples of 8 and 16) in the order the lanes of
+    dpk_fit_chain_f64 read it: entry (j, s, 16 g + c, u) is W[8 s + 2 g + u][16 j + c]."""
+    K, N = w.shape
+    return w.reshape(K // 8, 4, 2, N // 16, 16).permute(3, 0, 1, 4, 2).contiguous()
 
 
 def pack_fit_tail(hidden, wout, dtype=torch.bfloat16) -> np.ndarray:

@@ -570,6 +570,26 @@ int dpk_fit_layer_bwd(void* gy, void* gz, int prec, const void* mm,
                       const void* gy_next, const void* wvec, const void* sd,
                       int n, int h, int hnext, int res_next,
                       dpk_stream_t stream);
+/*
+ * The whole fitting of FP64 tanh nets in one call, every type segment
+ * in each launch (the math of the functions above, from xyz to dE/dxyz and
+ * the atomic energies).  Host arrays: widths [nlayers + 1] = d3 m2, h_1 ..
+ * h_L (each a multiple of 16; at most 8 layers); res [ntypes, nlayers] (0, 1,
+ * 2; 0 for the first layer); params [ntypes, 4 nlayers + 1] device addresses
+ * (64-bit): per layer W, W^T, b, idt (NULL: none), then w_out; ebias
+ * [ntypes]; segs [nseg, 3] = (type, first slot, end), in slot order without
+ * gaps (at most 16).  A weight [K, N] is laid out in fragments: value
+ * W[8 s + 2 g + u][16 j + c] at ((j (K / 8) + s) 64 + 16 g + c) 2 + u.
+ * desc [n, d3 m2] receives the descriptor; ws: workspace of
+ * dpk_fit_chain_f64_workspace_bytes.
+ */
+size_t dpk_fit_chain_f64_workspace_bytes(int n, int nlayers, const int* widths);
+int dpk_fit_chain_f64(int nlayers, const int* widths, const int* res,
+                      const void* const* params, const double* ebias, int nseg,
+                      const int* segs, double* atom_energy, double* gxyz,
+                      const double* xyz, const int* order, int n, int d3,
+                      int m2, double* desc, void* ws, size_t ws_bytes,
+                      dpk_stream_t stream);
 /* Fused BF16 fitting tail of one type segment, replacing, for nets of L = 2
  * or 3 hidden layers of width 256, the chain dpk_fit_layer_fwd (layer 1..L),
  * the layer 2..L GEMMs, dpk_fit_energy, the backward GEMMs of layers L..2

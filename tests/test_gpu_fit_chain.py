@@ -1,0 +1,67 @@
+"""The FP64 fitting in one call (csrc/fit_chain.hip): row counts around the 16-,
+32- and 64-row tiles, empty types, every resnet form, narrow and wide layers,
+against torch's FP64 autograd on the CPU."""
+
+import numpy as np
+import pytest
+import torch
+
+from deepmd_amd import model as M
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _torch_energy(layers, d):
+    x = d
+    for ly in layers[:-1]:
+        y = torch.tanh(x @ torch.tensor(ly.w) + torch.tensor(ly.b))
+        if ly.idt is not None:
+            y = y * torch.tensor(ly.idt)
+        r = M._res_mode(ly.w.shape[0], ly.w.shape[1], ly.resnet)
+        x = y + (x if r == 1 else torch.cat([x, x], -1) if r == 2 else 0.0)
+    return (x @ torch.tensor(layers[-1].w))[:, 0] + float(layers[-1].b[0])
+
+
+@pytest.mark.parametrize("widths,d3,m2,rows,dt", [
+    ([240, 240, 240], 100, 16, [27, 54], True),      # 16 x 16 tiles, K split
+    ([240, 240, 240], 100, 16, [513, 1000], True),   # 32 x 32 tiles
+    ([240, 240], 128, 16, [5000], False),            # 64 x 64 tiles
+    ([32, 64, 64], 64, 4, [1, 0, 17], True),         # resnet 2 and 1, an empty type
+    ([16], 32, 8, [33], False),                      # one layer
+    ([48, 48, 96], 40, 16, [16, 15, 2], True),
+    ([256, 256, 256], 128, 16, [64, 65], False),
+])
+def test_fit_chain_vs_autograd(widths, d3, m2, rows, dt):
+    rng = np.random.default_rng(5)
+    nt = len(rows)
+    nets = [M._layers(M._rand_net(rng, [d3 * m2] + widths + [1], dt, True)) for _ in range(nt)]
+    bias = rng.normal(size=nt)
+    fit = M.Fitting(nets, bias, np.zeros(nt), "f64", torch.device(DEV))
+    assert fit.chain is not None
+    n = sum(rows)
+    order = rng.permutation(n).astype(np.int32)
+    segs = [(t, sum(rows[:t]), sum(rows[:t + 1])) for t in range(nt)]
+    xyz = rng.normal(size=(n, 4, d3)) * 0.3
+    x = torch.tensor(xyz, device=DEV)
+    ae = torch.full((n,), float("nan"), dtype=torch.float64, device=DEV)
+    gx = torch.full((n, 4, d3), float("nan"), dtype=torch.float64, device=DEV)
+    fit.run(ae, gx, x, torch.tensor(order, device=DEV), segs, n, fit.buffers(n), d3, m2,
+            torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    ref = torch.tensor(xyz, requires_grad=True)
+    e = torch.zeros(n, dtype=torch.float64)
+    for t, a, b in segs:
+        if b == a:
+            continue
+        idx = torch.tensor(order[a:b].astype(np.int64))
+        xs = ref[idx]
+        d = torch.matmul(xs.transpose(1, 2), xs[:, :, :m2]).reshape(b - a, -1)
+        e = e.index_put((idx,), _torch_energy(nets[t], d) + bias[t])
+    g, = torch.autograd.grad(e.sum(), ref)
+    # sums of up to 2048 terms rounded at 1.1e-16, through a few layers: < 1e-12
+    # of the largest value
+    for name, got, want in (("energy", ae, e.detach()), ("gxyz", gx, g)):
+        err = float((got.cpu() - want).abs().max() / want.abs().max())
+        print(f"{name} {widths} {rows}: {err:.2e}", flush=True)
+        assert err < 1e-12, name
