@@ -273,11 +273,13 @@ __global__ void __launch_bounds__(64 * W) k_force_cells(
     const int* __restrict__ img_shift, const double* __restrict__ stdv,
     const int* __restrict__ cell_start, const int* __restrict__ cell_atoms,
     const int* __restrict__ atom_cell, const int* __restrict__ atom_slot, int nnei, double rcut,
-    double rcut_smth, double protection, const int* __restrict__ pair_mask, int ntypes) {
+    double rcut_smth, double protection, const int* __restrict__ pair_mask, int ntypes,
+    int parts) {
   __shared__ double tab[kCellTab * 3];
-  const int cell = blockIdx.x;
+  // `parts` workgroups share a cell's centres, W at a time in turn
+  const int cell = blockIdx.x / parts, first = (blockIdx.x % parts) * W;
   const int a0 = cell_start[cell], a1 = cell_start[cell + 1];
-  if (a1 <= a0) return;  // uniform over the workgroup
+  if (a1 <= a0 + first) return;  // uniform over the workgroup
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   for (int q = threadIdx.x; q < kCellTab * 3; q += blockDim.x) tab[q] = 0.0;
   const dpk_frame& fd = frames[frame_of[cell_atoms[a0]]];
@@ -289,7 +291,7 @@ __global__ void __launch_bounds__(64 * W) k_force_cells(
   bync2.init((unsigned)fd.nc[2]);
   bync1.init((unsigned)fd.nc[1]);
   __syncthreads();
-  for (int ai = a0 + wave; ai < a1; ai += W) {
+  for (int ai = a0 + first + wave; ai < a1; ai += W * parts) {
     const int g = cell_atoms[ai];
     const int traw = atype[g];
     const int ti = traw < 0 ? 0 : traw;
@@ -824,16 +826,21 @@ extern "C" int dpk_force_virial_cells(double* force, double* atom_virial, const 
   // cell unless set (DPK_TUNE_FORCE_WAVES).  16 only for very full cells: at
   // ~48 atoms per cell (FCC Cu, rcut 6) 8 wavefronts take 530 us where 16
   // take 625 us (two 41 KB workgroups of 16 fill a CU's 32 wave slots; three
-  // of 8 leave room for the next cell's start-up)
+  // of 8 leave room for the next cell's start-up); 4 only for nearly empty ones
+  // (13 atoms a cell on average, 96 frames of 24..768: 213 us with 8, 276 with 4)
   int nw = tune(DPK_TUNE_FORCE_WAVES);
-  if (nw == 0) nw = natoms >= 96 * ncells ? 16 : (natoms >= 16 * ncells ? 8 : 4);
+  if (nw == 0) nw = natoms >= 96 * ncells ? 16 : (natoms >= 6 * ncells ? 8 : 4);
   nw = nw <= 4 ? 4 : (nw <= 8 ? 8 : 16);
+  int dev = 0, ncu = 0;
+  DPK_HIP(hipGetDevice(&dev));
+  DPK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  const int parts = cell_parts(natoms, ncells, nw, 3 * ncu);  // three tables fit a CU's LDS
 #define DPK_FORCE_CELLS(GT, NW)                                                              \
-  hipLaunchKernelGGL((k_force_cells<GT, NW>), dim3(ncells), dim3(64 * NW), 0, st, force, vrow, \
+  hipLaunchKernelGGL((k_force_cells<GT, NW>), dim3(ncells * parts), dim3(64 * NW), 0, st, force, vrow, \
                      atom_virial, static_cast<const GT*>(net_deriv), coord_wrapped, atype,     \
                      frame_of, frames, nlist, shift_vec, img_shift, std, w.cell_start,         \
                      w.cell_atoms, w.atom_cell, w.atom_slot, nnei, rcut, rcut_smth,             \
-                     protection, pair_mask, ntypes)
+                     protection, pair_mask, ntypes, parts)
 #define DPK_FORCE_CELLS_W(GT)            \
   if (nw == 16) DPK_FORCE_CELLS(GT, 16); \
   else if (nw == 8) DPK_FORCE_CELLS(GT, 8); \

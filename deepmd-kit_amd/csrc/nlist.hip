@@ -541,13 +541,14 @@ __global__ void __launch_bounds__(64 * W) k_search_cells(
     const int* __restrict__ atom_cell, const int* __restrict__ cell_start,
     const int* __restrict__ cell_atoms, const int* __restrict__ img_pos,
     const double* __restrict__ shift_vec, double rcut, SelInfo si, int capb, bool packed,
-    int* __restrict__ nlist, int* __restrict__ status) {
+    int parts, int* __restrict__ nlist, int* __restrict__ status) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int c_kb[kBlockCells], c_pre[kBlockCells + 1], c_img[kBlockCells];
   __shared__ int wg_max;
-  const int cell = blockIdx.x;
+  // `parts` workgroups share a cell's centres, W at a time in turn
+  const int cell = blockIdx.x / parts, first = (blockIdx.x % parts) * W;
   const int a0 = cell_start[cell], a1 = cell_start[cell + 1];
-  if (a1 <= a0) return;  // uniform over the workgroup
+  if (a1 <= a0 + first) return;  // uniform over the workgroup
   if (threadIdx.x == 0) wg_max = 0;
   __syncthreads();
   int wmax = 0;
@@ -624,7 +625,7 @@ __global__ void __launch_bounds__(64 * W) k_search_cells(
   const int eb = index_bits(fd);
   FastDiv nloc_div;
   nloc_div.init((unsigned)fd.nloc);
-  for (int ai = a0 + wave; ai < a1; ai += W) {
+  for (int ai = a0 + first + wave; ai < a1; ai += W * parts) {
     const int g = cell_atoms[ai];
     int* out = nlist + (size_t)g * S;
     if (atype[g] < 0) {  // virtual centre: empty row (nlist.py:193-195)
@@ -679,21 +680,30 @@ int launch_search_w(const double* wrapped, const int* atype, const int* frame_of
                     const dpk_frame* frames, const int* atom_cell, const int* cell_start,
                     const int* cell_atoms, const int* img_pos, const double* shift_vec,
                     double rcut, const SelInfo& si, int natoms, int ncells, int* nlist,
-                    int* status, size_t budget, hipStream_t st) {
-  // staged candidates: ~1.25x the mean 27-cell neighbourhood, within the LDS budget
+                    int* status, size_t budget, int ncu, bool ragged, hipStream_t st) {
+  // staged candidates: ~1.25x the mean 27-cell neighbourhood (3x where frames
+  // may differ in how full their cells are), within the LDS budget
   const size_t wbytes = (size_t)W * search_wave_bytes<MAXC>(si.nnei);
   DPK_REQUIRE(wbytes + 64 * sizeof(BCand) <= budget, DPK_ERR_UNSUPPORTED,
               "nlist: candidate buffers of %zu bytes exceed the LDS budget %zu", wbytes, budget);
-  long want = (long)(27.0 * natoms / ncells * tune(DPK_TUNE_NLIST_STAGE_PCT) / 100.0) + 64;
+  const double pct = tune(DPK_TUNE_NLIST_STAGE_PCT) * (ragged ? 2.4 : 1.0);
+  long want = (long)(27.0 * natoms / ncells * pct / 100.0) + 64;
   long capb = (long)((budget - wbytes) / sizeof(BCand));
   if (want < capb) capb = want;
   capb = capb / 64 * 64;
   if (capb < 64) capb = 64;
   if (tune(DPK_TUNE_NLIST_MODE) == 1) capb = 0;  // every centre gathers from global memory
   const size_t lds = sizeof(BCand) * (size_t)(capb > 0 ? capb : 1) + wbytes;
-  hipLaunchKernelGGL((k_search_cells<MAXC, W>), dim3(ncells), dim3(64 * W), lds, st, wrapped,
-                     atype, frame_of, frames, atom_cell, cell_start, cell_atoms, img_pos,
-                     shift_vec, rcut, si, (int)capb, tune(DPK_TUNE_NLIST_SORT) == 0, nlist,
+  int parts = cell_parts(natoms, ncells, W, ncu);
+  // frames of different sizes: their fullest cells (a small box is one cell)
+  // decide, as far as the other cells' idle workgroups cost little
+  if (ragged && parts < 4) {
+    const int most = 8 * ncu / ncells < 4 ? 8 * ncu / ncells : 4;
+    parts = parts > most ? parts : most;
+  }
+  hipLaunchKernelGGL((k_search_cells<MAXC, W>), dim3(ncells * parts), dim3(64 * W), lds, st,
+                     wrapped, atype, frame_of, frames, atom_cell, cell_start, cell_atoms, img_pos,
+                     shift_vec, rcut, si, (int)capb, tune(DPK_TUNE_NLIST_SORT) == 0, parts, nlist,
                      status);
   DPK_LAUNCHED();
   return DPK_OK;
@@ -701,20 +711,26 @@ int launch_search_w(const double* wrapped, const int* atype, const int* frame_of
 
 // Wavefronts per cell workgroup: more of them share one staged neighbourhood
 // and hide the latency of the per-centre scan and sort (a workgroup of 16
-// takes a whole CU); fewer where cells hold few atoms.
+// takes a whole CU); fewer where cells hold few atoms (measured: 24 atoms a
+// cell, 12,288 in all, 8 wavefronts 68 us, 16 84; 32 a cell, 3,993 in all, 90
+// and 64).  Batches of frames take 16 from 8 atoms a cell on: their cells
+// differ, and the fullest -- a frame of one cell -- are the longest (96 frames
+// of 24..768 atoms: 4 wavefronts and 1.25x staged 534 us, 16 and 3x 291).
 template <int MAXC>
 int launch_search(const double* wrapped, const int* atype, const int* frame_of,
                   const dpk_frame* frames, const int* atom_cell, const int* cell_start,
                   const int* cell_atoms, const int* img_pos, const double* shift_vec,
                   double rcut, const SelInfo& si, int natoms, int ncells, int* nlist,
-                  int* status, hipStream_t st) {
+                  int* status, bool ragged, hipStream_t st) {
   int dev = 0, maxlds = 0;
   DPK_HIP(hipGetDevice(&dev));
   DPK_HIP(hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+  int ncu = 0;
+  DPK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
   const size_t budget = (size_t)(maxlds < 160 * 1024 ? maxlds : 160 * 1024) - 512;
   const double per_cell = (double)natoms / ncells;
   int w = tune(DPK_TUNE_NLIST_WAVES);
-  if (w == 0) w = per_cell >= 32.0 ? 16 : (per_cell >= 16.0 ? 8 : 4);
+  if (w == 0) w = per_cell >= (ragged ? 8.0 : 28.0) ? 16 : (per_cell >= 16.0 ? 8 : 4);
   w = w <= 4 ? 4 : (w <= 8 ? 8 : 16);
   // keep room for the per-wavefront buffers and a full mean neighbourhood
   const size_t stage = (size_t)(27.0 * per_cell + 64) * sizeof(BCand);
@@ -722,7 +738,7 @@ int launch_search(const double* wrapped, const int* atype, const int* frame_of,
 #define DPK_SEARCH_W(NW)                                                                        \
   return launch_search_w<MAXC, NW>(wrapped, atype, frame_of, frames, atom_cell, cell_start,     \
                                    cell_atoms, img_pos, shift_vec, rcut, si, natoms, ncells,    \
-                                   nlist, status, budget, st)
+                                   nlist, status, budget, ncu, ragged, st)
   if (w == 16) DPK_SEARCH_W(16);
   if (w == 8) DPK_SEARCH_W(8);
   DPK_SEARCH_W(4);
@@ -959,7 +975,7 @@ extern "C" int dpk_nlist_build(int* nlist, double* coord_wrapped, int* status_de
 #define DPK_SEARCH(M)                                                                       \
   return launch_search<M>(coord_wrapped, atype, frame_of, frames, atom_cell, cell_start,   \
                           cell_atoms, img_pos, shift_vec, rcut, si, natoms, ncells, nlist, \
-                          status_dev, st)
+                          status_dev, nframes > 1, st)
   if (max_cand <= 256) DPK_SEARCH(256);
   if (max_cand <= 512) DPK_SEARCH(512);
   if (max_cand <= 1024) DPK_SEARCH(1024);

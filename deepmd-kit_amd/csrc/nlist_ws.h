@@ -40,4 +40,16 @@ inline NlistWs nlist_ws(void* workspace, int natoms, int ncells) {
   return w;
 }
 
+// Workgroups that share a cell's centres (W wavefronts each): one where the
+// cells alone fill the chip, more -- down to a centre a wavefront -- where a
+// few cells hold all atoms (a small periodic box is one to eight cells).
+// Search and forces of 81 water atoms in one cell: 132 and 82 us with one
+// workgroup, 43 and 21 us with six and eleven; 5,324 Cu atoms in 64 cells: 128
+// and 119 us, 53 and 102 us.
+inline int cell_parts(int natoms, int ncells, int W, int ncu) {
+  const int rounds = (natoms + ncells * W - 1) / (ncells * W), room = ncu / ncells;
+  const int p = rounds < room ? rounds : room;
+  return p > 1 ? p : 1;
+}
+
 }  // namespace dpk
