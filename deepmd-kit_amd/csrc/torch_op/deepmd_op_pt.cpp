@@ -294,8 +294,9 @@ Tensor force_impl(const Tensor& net_deriv, const Tensor& in_deriv, const Tensor&
   TORCH_CHECK(net_deriv.numel() == nf * nloc * nnei * 4 && in_deriv.numel() == nf * nloc * nnei * 12,
               op, ": net_deriv / in_deriv do not match nlist");
   const c10::DeviceGuard guard(net_deriv.device());
-  Tensor force = torch::zeros({nf, nall * 3}, net_deriv.options().dtype(torch::kFloat64));
-  if (nf * nloc * nnei == 0) return force.to(net_deriv.scalar_type());
+  auto o64 = net_deriv.options().dtype(torch::kFloat64);
+  if (nf * nloc * nnei == 0) return torch::zeros({nf, nall * 3}, o64).to(net_deriv.scalar_type());
+  Tensor force = torch::empty({nf, nall * 3}, o64);  // (cleared by the call)
   Tensor g = f64c(net_deriv), d = f64c(in_deriv), n = i32c(nlist);
   check_rc(dpk_prod_force_a_f64(force.data_ptr<double>(), g.data_ptr<double>(),
                                 d.data_ptr<double>(), n.data_ptr<int>(), (int)nf, (int)nloc,
@@ -313,7 +314,8 @@ Tensor force_grad_impl(const Tensor& grad, const Tensor& in_deriv, const Tensor&
   TORCH_CHECK(grad.numel() == nf * ngrad * 3 && in_deriv.numel() == nf * nloc * nnei * 12, op,
               ": grad / in_deriv do not match nlist");
   const c10::DeviceGuard guard(grad.device());
-  Tensor gn = torch::zeros({nf, nloc * nnei * 4}, grad.options().dtype(torch::kFloat64));
+  // (the kernel writes every value)
+  Tensor gn = torch::empty({nf, nloc * nnei * 4}, grad.options().dtype(torch::kFloat64));
   if (nf * nloc * nnei == 0) return gn.to(out_dtype);
   Tensor g = f64c(grad), d = f64c(in_deriv), n = i32c(nlist);
   check_rc(dpk_prod_force_grad_a_f64(gn.data_ptr<double>(), g.data_ptr<double>(),
@@ -333,7 +335,8 @@ Tensor virial_grad_impl(const Tensor& grad, const Tensor& in_deriv, const Tensor
                   rij.numel() == nf * nloc * nnei * 3,
               op, ": grad / in_deriv / rij do not match nlist");
   const c10::DeviceGuard guard(grad.device());
-  Tensor gn = torch::zeros({nf, nloc * nnei * 4}, grad.options().dtype(torch::kFloat64));
+  // (the kernel writes every value)
+  Tensor gn = torch::empty({nf, nloc * nnei * 4}, grad.options().dtype(torch::kFloat64));
   if (nf * nloc * nnei == 0) return gn.to(out_dtype);
   Tensor g = f64c(grad), d = f64c(in_deriv), r = f64c(rij), n = i32c(nlist);
   check_rc(dpk_prod_virial_grad_a_f64(gn.data_ptr<double>(), g.data_ptr<double>(),
@@ -357,9 +360,10 @@ std::vector<Tensor> virial_impl(const Tensor& net_deriv, const Tensor& in_deriv,
               op, ": net_deriv / in_deriv / rij do not match nlist");
   const c10::DeviceGuard guard(net_deriv.device());
   auto o64 = net_deriv.options().dtype(torch::kFloat64);
-  Tensor vir = torch::zeros({nf, 9}, o64);
-  Tensor av = torch::zeros({nf, nall * 9}, o64);
-  if (nf * nloc * nnei > 0) {
+  const bool any = nf * nloc * nnei > 0;  // (then the call clears and writes both)
+  Tensor vir = any ? torch::empty({nf, 9}, o64) : torch::zeros({nf, 9}, o64);
+  Tensor av = any ? torch::empty({nf, nall * 9}, o64) : torch::zeros({nf, nall * 9}, o64);
+  if (any) {
     Tensor ws = torch::empty({(int64_t)dpk_prod_virial_workspace_bytes((int)nf, (int)nloc) + 8},
                              net_deriv.options().dtype(torch::kUInt8));
     Tensor g = f64c(net_deriv), d = f64c(in_deriv), r = f64c(rij), n = i32c(nlist);

@@ -294,11 +294,12 @@ def embed_internal(packed_k, s, r2, r3, act="tanh"):
     return act_np(act, y2 @ w3t.T + b3) * i3 + (np.tile(y2, 2) if r3 == 2 else 0.0)
 
 
-def padding_table(packed, net_of, davg, dstd, sec, r2, r3, act="tanh"):
+def padding_table(packed, net_of, davg, dstd, sec, r2, r3, act="tanh", distinct=False):
     """pad[ti, jj, c, k]: sum over the slots jj..end of jj's type block of
     R[c] G[k] for the padding rows R = (0 - davg) / dstd of centre type ti
     (G = their net at s = R[0], internal channel k), or None when every
-    padding row is zero (include/dpk.h, dpk_embed_fwd)."""
+    padding row is zero (include/dpk.h, dpk_embed_fwd).  ``distinct``: the net
+    runs once for equal rows (a block's are, but for unusual statistics)."""
     nt, nnei = davg.shape[0], davg.shape[1]
     R = -davg / dstd  # [nt, nnei, 4]
     if not np.any(R):
@@ -309,7 +310,10 @@ def padding_table(packed, net_of, davg, dstd, sec, r2, r3, act="tanh"):
             a, b = int(sec[t]), int(sec[t + 1])
             if b <= a:
                 continue
-            G = embed_internal(packed[net_of[ti, t]], R[ti, a:b, 0], r2, r3, act)  # [b-a, 128]
+            x, back = R[ti, a:b, 0], slice(None)
+            if distinct:
+                x, back = np.unique(x, return_inverse=True)
+            G = embed_internal(packed[net_of[ti, t]], x, r2, r3, act)[back]  # [b-a, 128]
             C = R[ti, a:b, :, None] * G[:, None, :]
             pad[ti, a:b] = np.cumsum(C[::-1], axis=0)[::-1]
     return pad
@@ -853,7 +857,7 @@ class SeAModel:
         if self.skip_padding:
             pad = padding_table(packed, net_of, self.davg.reshape(nt, self.nnei, 4),
                                 self.dstd.reshape(nt, self.nnei, 4), self.sec, r2, r3,
-                                self.emb_act_name)
+                                self.emb_act_name, distinct=self.precision == "f64")
             if pad is not None:
                 self.emb_pad = torch.tensor(pad, dtype=real, device=dev).contiguous()
         self.pair_mask = None  # (ntypes+1)^2 type-pair table, exclude_mask.py:64-140
@@ -1039,7 +1043,7 @@ class SeAModel:
         sysd.force = torch.empty((nall, 3), dtype=torch.float64, device=dev)
         sysd.vrow = torch.empty(int(lib.dpk_force_virial_workspace_bytes(nloc)), dtype=torch.uint8,
                                 device=dev)
-        # inverted list + per-slot force shares of dpk_force_virial_gather
+        # (dpk_force_virial_gather's workspace)
         sysd.extra["ws_gather"] = torch.empty(
             int(lib.dpk_force_virial_gather_workspace_bytes(nloc, S, nall)), dtype=torch.uint8,
             device=dev)
@@ -1202,7 +1206,7 @@ class SeAModel:
         if atomic_virial:
             av = torch.empty((nall, 9), dtype=torch.float64, device=s.force.device)
         if nloc:
-            # neighbour forces gathered per extended atom (no atomics)
+            # neighbour forces added to the extended atoms' rows
             wg = s.extra["ws_gather"]
             call("dpk_force_virial_gather", ptr(s.force), ptr(av), ptr(s.vrow), ptr(s.nd),
                  self.prec, ptr(s.coord), ptr(s.atype), ptr(s.nlist), ptr(self.dstd_dev), nloc,

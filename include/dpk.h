@@ -671,12 +671,10 @@ int dpk_force_virial_fused(double* force, double* atom_virial, const void* net_d
 /*
  * Forces and virial of an engine's extended region (the MD-engine path:
  * explicit ghosts, nlist [natoms, nnei] of extended-atom indices in
- * [0, nall), coord = the extended coordinates [nall, 3]) with the
- * neighbour sums gathered, not added with FP64 atomics: per call the slots
- * are binned by neighbour into fixed-capacity buckets (slots beyond a full
- * bucket are added with atomics at the end), a first pass writes each slot's
- * neighbour share and the centre's own force, a second pass sums every
- * extended atom's bucket.
+ * [0, nall), coord = the extended coordinates [nall, 3]): one pass over the
+ * slots, whose shares are added to their neighbours' rows with FP64 atomics,
+ * three consecutive lanes a row.  The workspace is not read or written (its
+ * size is a formality of earlier forms).
  * force [nall, 3] and atom_virial [nall, 9] (optional, NULL to skip; the
  * neighbour rows, as dpk_force_virial_fused) are overwritten; vrow
  * [natoms, 9] receives the per-centre virial rows (reduce with
