@@ -31,7 +31,8 @@
 //
 // Precision: F32 (v_mfma_f32_16x16x4_f32) runs the policy kernels below; BF16
 // / FP16 (FP32 accumulate, FP32 activations) have their own kernels in
-// namespace bf (LDS-resident weights, K = 32 MFMA); FP64 is in embed_f64.hip.
+// namespace bf (LDS-resident weights, K = 32 MFMA); FP16X2 is in
+// embed_f16x2.hip, FP64 in embed_f64.hip.
 #include <type_traits>
 
 #include "dpk_common.h"
@@ -40,6 +41,11 @@
 
 namespace dpk {
 
+// embed_f16x2.hip
+int embed_f16x2(bool fwd, void* out, const void* em, const void* gx, const int* atype,
+                const void* image, const int* net_of, const int* ch_out, int ntypes, int nnets,
+                int res2, int res3, int has_idt, int d3, const int* sec_host, int natoms,
+                int nnei, const int* nlist, const float* pad, hipStream_t st);
 // embed_f64.hip
 int embed_f64(bool fwd, void* out, const void* em, const void* gx, const int* atype,
               const void* params, const int* net_of, const int* ch_out, int ntypes, int nnets,
@@ -465,25 +471,6 @@ __device__ __forceinline__ v2u pack4(float a0, float a1, float a2, float a3) {
   return v2u{E::pack2(a0, a1), E::pack2(a2, a3)};
 }
 
-// Low parts of split operands (E::kSplit, FP16): lo = fp16(x - hi) for the
-// values packed in hi.
-__device__ __forceinline__ unsigned lo_pair(float a, float b, unsigned hi) {
-  return h16::F16::pack2(h16::sub_f16_lo(a, hi), h16::sub_f16_hi(b, hi));
-}
-
-template <class E>
-__device__ __forceinline__ v4u lo8(const float a[4], const float b[4], v4u hi) {
-  static_assert(E::kSplit, "split operands are FP16");
-  return v4u{lo_pair(a[0], a[1], hi[0]), lo_pair(a[2], a[3], hi[1]), lo_pair(b[0], b[1], hi[2]),
-             lo_pair(b[2], b[3], hi[3])};
-}
-
-template <class E>
-__device__ __forceinline__ v2u lo4(float a0, float a1, float a2, float a3, v2u hi) {
-  static_assert(E::kSplit, "split operands are FP16");
-  return v2u{lo_pair(a0, a1, hi[0]), lo_pair(a2, a3, hi[1])};
-}
-
 __device__ __forceinline__ v4u lds8(const unsigned char* p) {
   return *reinterpret_cast<const v4u*>(p);
 }
@@ -504,14 +491,12 @@ __device__ __forceinline__ void stage(unsigned char* dst, const unsigned char* s
 // operands are packed as d / K (one multiply per packed value), so the MFMA
 // returns the true W d and the tangents stay true derivatives.
 
-// Scaled 16-bit operand of the tangent MFMAs (and its low part when split).
+// Scaled 16-bit operand of the tangent MFMAs.
 template <class E>
-__device__ __forceinline__ v4u pack8_tangent(const float a[4], const float b[4], v4u* lo = nullptr) {
+__device__ __forceinline__ v4u pack8_tangent(const float a[4], const float b[4]) {
   const float as[4] = {a[0] * kInvK2L2E, a[1] * kInvK2L2E, a[2] * kInvK2L2E, a[3] * kInvK2L2E};
   const float bs[4] = {b[0] * kInvK2L2E, b[1] * kInvK2L2E, b[2] * kInvK2L2E, b[3] * kInvK2L2E};
-  const v4u hi = pack8<E>(as, bs);
-  if constexpr (E::kSplit) *lo = lo8<E>(as, bs, hi);
-  return hi;
+  return pack8<E>(as, bs);
 }
 
 // Layers 1-2 for the lane's slot: y1 (and dy1/ds) in registers, y2 (and dy2/ds).
@@ -542,19 +527,14 @@ __device__ __forceinline__ void layers12(const unsigned char* nb, float s, int g
       }
     }
   const v4u B1 = pack8<E>(y1[0], y1[1]);
-  v4u B1l, D1, D1l;
-  if constexpr (E::kSplit) B1l = lo8<E>(y1[0], y1[1], B1);
-  if (TANGENT) D1 = pack8_tangent<E>(d1[0], d1[1], &D1l);
+  v4u D1;
+  if (TANGENT) D1 = pack8_tangent<E>(d1[0], d1[1]);
 #pragma unroll
   for (int m = 0; m < 4; ++m) {
     const v4u a = lds8(nb + OFF_W2 + ((16 * m + c) * W2S + 8 * g) * 2);
     v4f acc = E::mfma32(a, B1, *reinterpret_cast<const v4f*>(vec + V_B2K + 16 * m + 4 * g));
-    if constexpr (E::kSplit) acc = E::mfma32(a, B1l, acc);
     v4f dacc;
-    if (TANGENT) {
-      dacc = E::mfma32(a, D1, v4f{0.f, 0.f, 0.f, 0.f});
-      if constexpr (E::kSplit) dacc = E::mfma32(a, D1l, dacc);
-    }
+    if (TANGENT) dacc = E::mfma32(a, D1, v4f{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int ch = 16 * m + 4 * g + i;
@@ -583,7 +563,6 @@ __device__ __forceinline__ void layers12(const unsigned char* nb, float s, int g
 template <class E, bool TANGENT, class C>
 __device__ __forceinline__ void layer3_block(const unsigned char* nb, int m, int g, int c,
                                              const v4u B2[2], const v4u D2[2],
-                                             const v4u B2l[2], const v4u D2l[2],
                                              const float y2[4][4], const float d2[4][4],
                                              float G[4], float dG[4]) {
   const float* vec = reinterpret_cast<const float*>(nb);
@@ -591,18 +570,10 @@ __device__ __forceinline__ void layer3_block(const unsigned char* nb, int m, int
   const v4u a0 = lds8(row), a1 = lds8(row + 64);
   v4f acc = E::mfma32(a0, B2[0], *reinterpret_cast<const v4f*>(vec + V_B3K + 16 * m + 4 * g));
   acc = E::mfma32(a1, B2[1], acc);
-  if constexpr (E::kSplit) {
-    acc = E::mfma32(a0, B2l[0], acc);
-    acc = E::mfma32(a1, B2l[1], acc);
-  }
   v4f dacc;
   if (TANGENT) {
     dacc = E::mfma32(a0, D2[0], v4f{0.f, 0.f, 0.f, 0.f});
     dacc = E::mfma32(a1, D2[1], dacc);
-    if constexpr (E::kSplit) {
-      dacc = E::mfma32(a0, D2l[0], dacc);
-      dacc = E::mfma32(a1, D2l[1], dacc);
-    }
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -675,51 +646,28 @@ __global__ void __launch_bounds__(256) k_fwd(
         asm volatile("" ::: "memory");
         const int slot = s0 + c;
         const float s = slot < b1 ? e[slot * 4] : 0.f;
-        // A operand R^T: rows 0-3 the env-matrix components; split operands
-        // put their lo parts in rows 4-7, so one MFMA forms R_hi G and R_lo G
-        // (the two row groups are summed once per atom)
+        // A operand R^T: rows 0-3 the env-matrix components
         float rr[4];
-        constexpr int kRows = E::kSplit ? 8 : 4;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int sl = s0 + 4 * g + i;
-          rr[i] = (c < kRows && sl < b1) ? e[sl * 4 + (c & 3)] : 0.f;
+          rr[i] = (c < 4 && sl < b1) ? e[sl * 4 + c] : 0.f;
         }
-        v2u rT = pack4<E>(rr[0], rr[1], rr[2], rr[3]);
-        if constexpr (E::kSplit) {
-          const v2u rl = lo4<E>(rr[0], rr[1], rr[2], rr[3], rT);
-          if (c >= 4) rT = rl;
-        }
+        const v2u rT = pack4<E>(rr[0], rr[1], rr[2], rr[3]);
         float y1[2][4], d1[2][4], y2[4][4], d2[4][4];
         layers12<E, false, C>(nb, s, g, c, y1, d1, y2, d2);
         const v4u B2[2] = {pack8<E>(y2[0], y2[1]), pack8<E>(y2[2], y2[3])};
-        v4u B2l[2];
-        if constexpr (E::kSplit) {
-          B2l[0] = lo8<E>(y2[0], y2[1], B2[0]);
-          B2l[1] = lo8<E>(y2[2], y2[3], B2[1]);
-        }
 #pragma unroll
         for (int m = 0; m < 8; ++m) {
           float G[4], dG[4];
-          layer3_block<E, false, C>(nb, m, g, c, B2, B2, B2l, B2l, y2, d2, G, dG);
+          layer3_block<E, false, C>(nb, m, g, c, B2, B2, y2, d2, G, dG);
           // re-lay G with channels on lanes (identity), then R^T G over slots
           const v2u gh = pack4<E>(G[0], G[1], G[2], G[3]);
           const v4f gt = E::mfma16(gh, ident, v4f{0.f, 0.f, 0.f, 0.f});
           const v2u bt = pack4<E>(gt[0], gt[1], gt[2], gt[3]);  // exact: gt holds 16-bit values
           acc[m] = E::mfma16(rT, bt, acc[m]);
-          if constexpr (E::kSplit) {
-            const v4f gl = E::mfma16(lo4<E>(G[0], G[1], G[2], G[3], gh), ident,
-                                     v4f{0.f, 0.f, 0.f, 0.f});
-            acc[m] = E::mfma16(rT, pack4<E>(gl[0], gl[1], gl[2], gl[3]), acc[m]);
-          }
         }
       }
-    }
-    if constexpr (E::kSplit) {  // rows 4-7 (lo parts of R) onto rows 0-3
-#pragma unroll
-      for (int m = 0; m < 8; ++m)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[m][i] += __shfl_xor(acc[m][i], 16, 64);
     }
     if (valid && g == 0) {
       const float inv = 1.0f / (float)nnei;
@@ -736,7 +684,7 @@ __global__ void __launch_bounds__(256) k_fwd(
 }
 
 template <class E, bool RESIDENT, class C>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(E::kSplit ? 4 : 5))) k_bwd(
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_bwd(
     float* __restrict__ net_deriv, const float* __restrict__ em, const float* __restrict__ gxyz,
     const int* __restrict__ atype, const unsigned char* __restrict__ nets,
     const int* __restrict__ net_of, const int* __restrict__ ch_out, BlockInfo bi,
@@ -769,10 +717,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(E::kSp
     const float q = h16::pow2_scale(amax / (float)nnei);
     const float qin = q / (float)nnei;
     const float unq = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(1.0f / q)));
-    // rows 0-3 the components; split operands put their lo parts in rows
-    // 4-7, so one MFMA forms gx_hi B and gx_lo B (row groups summed per tile)
-    constexpr int kRows = E::kSplit ? 8 : 4;
-    const int comp = c & 3;
     v4u gxa[4];
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
@@ -780,17 +724,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(E::kSp
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         lo[i] = hi[i] = 0.f;
-        if (c < kRows && valid) {
+        if (c < 4 && valid) {
           const int t0 = ch_out[32 * p + 4 * g + i], t1 = ch_out[32 * p + 16 + 4 * g + i];
-          if (t0 >= 0) lo[i] = gxyz[aoff * 4 * d3 + comp * d3 + t0] * qin;
-          if (t1 >= 0) hi[i] = gxyz[aoff * 4 * d3 + comp * d3 + t1] * qin;
+          if (t0 >= 0) lo[i] = gxyz[aoff * 4 * d3 + c * d3 + t0] * qin;
+          if (t1 >= 0) hi[i] = gxyz[aoff * 4 * d3 + c * d3 + t1] * qin;
         }
       }
       gxa[p] = pack8<E>(lo, hi);
-      if constexpr (E::kSplit) {
-        const v4u l = lo8<E>(lo, hi, gxa[p]);
-        if (c >= 4) gxa[p] = l;
-      }
     }
     for (int t = 0; t < bi.ntypes; ++t) {
       const unsigned char* nb =
@@ -810,52 +750,25 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(E::kSp
         float y1[2][4], d1[2][4], y2[4][4], d2[4][4];
         layers12<E, true, C>(nb, s, g, c, y1, d1, y2, d2);
         const v4u B2[2] = {pack8<E>(y2[0], y2[1]), pack8<E>(y2[2], y2[3])};
-        v4u B2l[2], D2l[2];
-        const v4u D2[2] = {pack8_tangent<E>(d2[0], d2[1], &D2l[0]),
-                           pack8_tangent<E>(d2[2], d2[3], &D2l[1])};
-        if constexpr (E::kSplit) {
-          B2l[0] = lo8<E>(y2[0], y2[1], B2[0]);
-          B2l[1] = lo8<E>(y2[2], y2[3], B2[1]);
-        }
+        const v4u D2[2] = {pack8_tangent<E>(d2[0], d2[1]), pack8_tangent<E>(d2[2], d2[3])};
         v4f dR = {0.f, 0.f, 0.f, 0.f}, Mx = {0.f, 0.f, 0.f, 0.f}, Mr = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
           float G0[4], dG0[4], G1[4], dG1[4];
-          layer3_block<E, true, C>(nb, 2 * p, g, c, B2, D2, B2l, D2l, y2, d2, G0, dG0);
-          layer3_block<E, true, C>(nb, 2 * p + 1, g, c, B2, D2, B2l, D2l, y2, d2, G1, dG1);
+          layer3_block<E, true, C>(nb, 2 * p, g, c, B2, D2, y2, d2, G0, dG0);
+          layer3_block<E, true, C>(nb, 2 * p + 1, g, c, B2, D2, y2, d2, G1, dG1);
           const v4u gh = pack8<E>(G0, G1), dgh = pack8<E>(dG0, dG1);
           dR = E::mfma32(gxa[p], gh, dR);    // dR[comp][slot c]
           Mx = E::mfma32(gxa[p], dgh, Mx);   // sum_k gx[comp][k] dG[slot][k]
-          if constexpr (E::kSplit) {  // (gx_hi, gx_lo) x the lo parts
-            dR = E::mfma32(gxa[p], lo8<E>(G0, G1, gh), dR);
-            Mx = E::mfma32(gxa[p], lo8<E>(dG0, dG1, dgh), Mx);
-          }
           if constexpr (C::RES3 == 2) {
             // resnet copies (y2, y2) and (dy2, dy2): channels 32 p.. of G
             // repeat those of B2 / D2 [p & 1] (D2 holds dy2 / K)
             dR = E::mfma32(gxa[p], B2[p & 1], dR);
             Mr = E::mfma32(gxa[p], D2[p & 1], Mr);
-            if constexpr (E::kSplit) {
-              dR = E::mfma32(gxa[p], B2l[p & 1], dR);
-              Mr = E::mfma32(gxa[p], D2l[p & 1], Mr);
-            }
           }
           __builtin_amdgcn_sched_barrier(0);
         }
-        if constexpr (E::kSplit) {
-          // lanes g = 1 hold rows 4-7 (the gx_lo products): fold them into
-          // ds and dR of the lanes g = 0 (the components are the same)
-          float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
-          if (g < 2 && slot < b1) r = *reinterpret_cast<const float4*>(e + slot * 4);
-          float ds = r.x * (Mx[0] + K2L2E * Mr[0]) + r.y * (Mx[1] + K2L2E * Mr[1]) +
-                     r.z * (Mx[2] + K2L2E * Mr[2]) + r.w * (Mx[3] + K2L2E * Mr[3]);
-          ds += __shfl_xor(ds, 16, 64);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) dR[i] += __shfl_xor(dR[i], 16, 64);
-          if (g == 0 && slot < b1)
-            *reinterpret_cast<float4*>(nd + slot * 4) =
-                make_float4((dR[0] + ds) * unq, dR[1] * unq, dR[2] * unq, dR[3] * unq);
-        } else if (g == 0 && slot < b1) {
+        if (g == 0 && slot < b1) {
           const float4 r = *reinterpret_cast<const float4*>(e + slot * 4);
           const float ds = r.x * (Mx[0] + K2L2E * Mr[0]) + r.y * (Mx[1] + K2L2E * Mr[1]) +
                            r.z * (Mx[2] + K2L2E * Mr[2]) + r.w * (Mx[3] + K2L2E * Mr[3]);
@@ -1115,14 +1028,10 @@ int embed_common(bool fwd, void* out, int prec, const void* em, const void* gx,
       return bf::launch_cfg<h16::F16, false>(fwd, out, em, gx, atype, image, net_of, ch_out, bi,
                                              res2, res3, has_idt, nnets, d3, natoms, nnei, st);
     }
-    case DPK_PREC_F16X2: {  // the image of dpk_embed_pack_f16 (FP16 weights)
-      if ((size_t)nnets * bf::NET_BYTES <= (size_t)bf::kResidentMaxBytes)
-        return bf::launch_cfg<h16::F16x2, true>(fwd, out, em, gx, atype, image, net_of, ch_out,
-                                                bi, res2, res3, has_idt, nnets, d3, natoms, nnei,
-                                                st);
-      return bf::launch_cfg<h16::F16x2, false>(fwd, out, em, gx, atype, image, net_of, ch_out, bi,
-                                               res2, res3, has_idt, nnets, d3, natoms, nnei, st);
-    }
+    case DPK_PREC_F16X2:  // the image of dpk_embed_pack_f16 (FP16 weights)
+      return embed_f16x2(fwd, out, em, gx, atype, image, net_of, ch_out, ntypes, nnets, res2, res3,
+                         has_idt, d3, sec_host, natoms, nnei, nlist, static_cast<const float*>(pad),
+                         st);
     case DPK_PREC_F32:
       return launch_embed_cfg<PolF32>(fwd, out, em, gx, atype, params, net_of, ch_out, bi, res2,
                                       res3, has_idt, d3, natoms, nnei, st);

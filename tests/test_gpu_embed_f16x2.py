@@ -1,0 +1,83 @@
+"""FP16X2 embedding kernels (csrc/embed_f16x2.hip) on their own, against the
+oracle's descriptor contraction and its autograd: resnet and time-step variants,
+nets in LDS and read from memory, block lengths around the 16-slot tile."""
+
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+import torch
+
+from deepmd_amd.model import SeAModel, random_model_dict
+from oracle import sea
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+# The weights are FP16 values (below), so what is left is the split operands'
+# 2^-22 and FP32's tanh (1e-7), grown by a factor of about two a layer, and FP32
+# sums of up to 200 slots: below 1e-5 of the largest value; a lost low part
+# would be 2^-11 = 5e-4.
+TOL = 2e-5
+K = 2.8853900817779268  # the kernels' weights are rounded after this scaling
+
+
+def _case(neuron, sel, one_side, natoms, dt, seed=5):
+    d = random_model_dict(seed, 6.0, 0.5, sel, neuron, 4, [16, 16], type_one_side=one_side,
+                          resnet_dt_emb=dt, activation="tanh", fitting_activation="tanh")
+    de = d["model"]["descriptor"]
+    nt, nnei = len(sel), sum(sel)
+    rng = np.random.default_rng(seed + 1)
+    davg = np.zeros((nt, nnei, 4))
+    davg[..., 0] = 0.3 * (1 + np.arange(nt)[:, None])
+    de["@variables"]["davg"]["value"] = davg.tolist()
+    de["@variables"]["dstd"]["value"] = np.full((nt, nnei, 4), 0.5).tolist()
+    for net in de["embeddings"]["networks"]:
+        for ly in net["layers"][1:]:
+            w = ly["@variables"]["w"]
+            h = (np.asarray(w["value"], np.float32) * np.float32(K)).astype(np.float16)
+            w["value"] = (h.astype(np.float64) / K).tolist()
+    at = rng.integers(0, nt, natoms).astype(np.int32)
+    em = rng.normal(size=(natoms, nnei, 4)).astype(np.float32)
+    nl = np.zeros((natoms, nnei), dtype=np.int32)
+    sec = np.concatenate([[0], np.cumsum(sel)])
+    for i in range(natoms):
+        for t in range(nt):
+            real = rng.integers(0, sel[t] + 1) if i > 2 else (sel[t], 0, sel[t] // 2)[i]
+            nl[i, sec[t] + real:sec[t + 1]] = -1
+            em[i, sec[t] + real:sec[t + 1]] = -davg[at[i], 0] / 0.5
+    gx = (1e-3 * rng.normal(size=(natoms, 4, neuron[-1]))).astype(np.float32)
+    return d, at, em, nl, gx
+
+
+@pytest.mark.parametrize("neuron,sel,one_side,natoms,dt", [
+    ([25, 50, 100], [46, 92], True, 7, False),      # two nets in LDS
+    ([32, 64, 128], [200], True, 1100, False),
+    ([25, 50, 100], [17, 15], False, 41, False),    # four nets, read from memory
+    ([25, 50, 100], [16], True, 1, True),
+    ([10, 20, 40], [1, 31], True, 9, True),
+    ([20, 30, 100], [40], True, 50, False),         # no doubling: no resnet
+    ([20, 40, 100], [33], True, 4300, False),       # resnet of layer 2 only
+    ([20, 50, 100], [15, 16, 17], False, 30, True),  # of layer 3 only, nine nets
+])
+def test_embed_f16x2_vs_oracle(neuron, sel, one_side, natoms, dt):
+    d, at, em, nl, gx = _case(neuron, sel, one_side, natoms, dt)
+    om = sea.model_from_serialized(d)
+    e = torch.tensor(em, dtype=torch.float64, requires_grad=True)
+    _, xyz = sea.descriptor_from_env(om, e, torch.tensor(at).long(),
+                                     torch.ones(em.shape[:2], dtype=torch.int32))
+    nd, = torch.autograd.grad((xyz * torch.tensor(gx)).sum(), e)
+    nd = np.where((nl < 0)[..., None], 0.0, nd.numpy())
+    m = SeAModel(d, "f16x2", DEV)
+    to = lambda a: torch.tensor(a, device=DEV).contiguous()  # noqa: E731
+    nan = lambda *s: torch.full(s, float("nan"), device=DEV)  # noqa: E731
+    s = SimpleNamespace(fs=SimpleNamespace(natoms=natoms), em=to(em), atype=to(at), nlist=to(nl),
+                        gxyz=to(gx), xyz=nan(natoms, 4, m.d3), nd=nan(*em.shape))
+    st = torch.cuda.current_stream().cuda_stream
+    m._embed_forward(s, st)
+    m._embed_backward(s, st)
+    torch.cuda.synchronize()
+    for got, ref, what in ((s.xyz, xyz.detach().numpy(), "xyz"), (s.nd, nd, "net_deriv")):
+        err = np.max(np.abs(got.cpu().numpy() - ref)) / np.max(np.abs(ref))
+        print(f"{what} {neuron} {sel} n={natoms}: {err:.2e}", flush=True)
+        assert err < TOL, what
