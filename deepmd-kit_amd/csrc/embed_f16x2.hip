@@ -25,7 +25,8 @@
 // 131,072 Cu atoms (12 tiles an atom) forward 2.47 -> 2.30 ms, backward 3.79 ->
 // 3.64; three wavefronts a SIMD for the backward without its 32 bytes of
 // scratch (outside the loop) 3.74, five for the forward 2.32.
-// One wavefront an atom, 16 slots a tile; lane (g = lane / 16, c = lane % 16).
+// One wavefront an atom, or several where atoms are few (split_of), 16 slots a
+// tile; lane (g = lane / 16, c = lane % 16).
 #include "dpk_common.h"
 #include "half16.h"
 #include "embed_image.h"
@@ -173,7 +174,7 @@ template <bool RESIDENT, class C>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_fwd2(
     float* __restrict__ xyz, const float* __restrict__ em, const int* __restrict__ atype,
     const unsigned char* __restrict__ nets, const int* __restrict__ net_of,
-    const int* __restrict__ ch_out, Block2 bi, int nnets, int d3, int natoms, int nnei) {
+    const int* __restrict__ ch_out, Block2 bi, int nnets, int d3, int natoms, int nnei, int lp) {
   extern __shared__ __align__(16) unsigned char lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
@@ -181,8 +182,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
   const float id[4] = {c == 4 * g ? 1.f : 0.f, c == 4 * g + 1 ? 1.f : 0.f,
                        c == 4 * g + 2 ? 1.f : 0.f, c == 4 * g + 3 ? 1.f : 0.f};
   const v2u ident = pack4(id);
-  for (int base = blockIdx.x * 4; base < natoms; base += gridDim.x * 4) {
-    const int atom = base + wave;
+  // 1 << lp wavefronts an atom, each with every (1 << lp)-th tile
+  const int apw = 4 >> lp, part = wave & ((1 << lp) - 1);
+  for (int base = blockIdx.x * apw; base < natoms; base += gridDim.x * apw) {
+    const int atom = base + (wave >> lp);
     const bool valid = atom < natoms;
     int ti = valid ? atype[atom] : 0;
     ti = ti < 0 ? 0 : ti;
@@ -194,6 +197,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
     for (int m = 0; m < 8; ++m) acc[m] = kZero4;
 #pragma unroll
     for (int m = 0; m < 4; ++m) accY[m] = kZero4;
+    int tix = 0;  // tiles of the blocks before this one
     for (int t = 0; t < bi.ntypes; ++t) {
       const int net = net_of[ti * bi.ntypes + t];
       const unsigned char* nb = RESIDENT ? lds + (size_t)net * (NET_BYTES + kBias4)
@@ -204,7 +208,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
       if (bi.nlist != nullptr && valid) {
         b1 = block_end(bi.nlist + (size_t)atom * nnei, b0, b1, lane);
         // a virtual centre's rows are zero, not padding rows
-        if (bi.pad != nullptr && b1 < bi.sec[t + 1] && g == 0 && atype[atom] >= 0) {
+        if (bi.pad != nullptr && b1 < bi.sec[t + 1] && part == 0 && g == 0 && atype[atom] >= 0) {
           const float* pt = bi.pad + ((size_t)ti * nnei + b1) * 4 * P3;
 #pragma unroll
           for (int m = 0; m < 8; ++m)
@@ -212,7 +216,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
             for (int i = 0; i < 4; ++i) acc[m][i] -= 0.5f * pt[i * P3 + 16 * m + c];
         }
       }
-      for (int s0 = b0; s0 < b1; s0 += 16) {
+      const int first = (part - tix) & ((1 << lp) - 1);
+      tix += (b1 - b0 + 15) >> 4;
+      for (int s0 = b0 + 16 * first; s0 < b1; s0 += 16 << lp) {
         // weights are re-read from LDS every tile rather than hoisted into
         // registers across the loop (that would halve the occupancy)
         asm volatile("" ::: "memory");
@@ -269,18 +275,37 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
         }
       }
     }
-    const float inv = 1.0f / (float)nnei;
-    float* o = xyz + (size_t)(valid ? atom : 0) * 4 * d3;
+    float* part_lds = reinterpret_cast<float*>(lds + (RESIDENT ? nnets * (NET_BYTES + kBias4) : 0));
 #pragma unroll
-    for (int m = 0; m < 8; ++m) {
-      const int tc = ch_out[16 * m + c];
+    for (int m = 0; m < 8; ++m)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         float v = __builtin_fmaf(-2.0f, acc[m][i], accS[i] + accY[m & 3][i]);
-        v += __shfl_xor(v, 16, 64);
-        if (valid && g == 0 && tc >= 0) o[i * d3 + tc] = v * inv;
+        acc[m][i] = v + __shfl_xor(v, 16, 64);
       }
+    if (lp > 0) {  // the other wavefronts' sums, in their order
+      __syncthreads();
+      if (g == 0)
+#pragma unroll
+        for (int m = 0; m < 8; ++m)
+          *reinterpret_cast<v4f*>(part_lds + ((wave * 8 + m) * 16 + c) * 4) = acc[m];
+      __syncthreads();
+      if (part == 0 && g == 0)
+        for (int w = wave + 1; w < wave + (1 << lp); ++w)
+#pragma unroll
+          for (int m = 0; m < 8; ++m)
+            acc[m] += *reinterpret_cast<const v4f*>(part_lds + ((w * 8 + m) * 16 + c) * 4);
     }
+    const float inv = 1.0f / (float)nnei;
+    float* o = xyz + (size_t)(valid ? atom : 0) * 4 * d3;
+    if (valid && part == 0 && g == 0)
+#pragma unroll
+      for (int m = 0; m < 8; ++m) {
+        const int tc = ch_out[16 * m + c];
+        if (tc >= 0)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i * d3 + tc] = acc[m][i] * inv;
+      }
   }
 }
 
@@ -289,12 +314,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
     float* __restrict__ net_deriv, const float* __restrict__ em, const float* __restrict__ gxyz,
     const int* __restrict__ atype, const unsigned char* __restrict__ nets,
     const int* __restrict__ net_of, const int* __restrict__ ch_out, Block2 bi, int nnets, int d3,
-    int natoms, int nnei) {
+    int natoms, int nnei, int lp) {
   extern __shared__ __align__(16) unsigned char lds[];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   if (RESIDENT) stage<false>(lds, nets, nnets);
-  for (int base = blockIdx.x * 4; base < natoms; base += gridDim.x * 4) {
-    const int atom = base + wave;
+  // 1 << lp wavefronts an atom, each with every (1 << lp)-th tile
+  const int apw = 4 >> lp, part = wave & ((1 << lp) - 1);
+  for (int base = blockIdx.x * apw; base < natoms; base += gridDim.x * apw) {
+    const int atom = base + (wave >> lp);
     const bool valid = atom < natoms;
     int ti = valid ? atype[atom] : 0;
     ti = ti < 0 ? 0 : ti;
@@ -350,6 +378,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
       }
       if constexpr (!C::IDT) S = E::mfma32(gxa[p], v4u{kOne2, kOne2, kOne2, kOne2}, S);
     }
+    int tix = 0;  // tiles of the blocks before this one
     for (int t = 0; t < bi.ntypes; ++t) {
       const unsigned char* nb =
           (RESIDENT ? lds : nets) + (size_t)net_of[ti * bi.ntypes + t] * NET_BYTES;
@@ -359,10 +388,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
       if (bi.nlist != nullptr && valid) {
         // slots after the last real neighbour move no atom: dE/d em = 0
         b1 = block_end(bi.nlist + (size_t)atom * nnei, b0, b1, lane);
-        for (int z = b1 + lane; z < bi.sec[t + 1]; z += 64)
+        for (int z = b1 + lane + 64 * part; z < bi.sec[t + 1]; z += 64 << lp)
           *reinterpret_cast<float4*>(nd + z * 4) = make_float4(0.f, 0.f, 0.f, 0.f);
       }
-      for (int s0 = b0; s0 < b1; s0 += 16) {
+      const int first = (part - tix) & ((1 << lp) - 1);
+      tix += (b1 - b0 + 15) >> 4;
+      for (int s0 = b0 + 16 * first; s0 < b1; s0 += 16 << lp) {
         asm volatile("" ::: "memory");
         const int slot = s0 + c;
         const float s = slot < b1 ? e[slot * 4] : 0.f;
@@ -437,29 +468,46 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
 }
 
 constexpr int kResidentMaxBytes = 64 * 1024;
+constexpr int kPartSums = 4 * 8 * 16 * 16;  // forward, split atoms: four wavefronts' sums
+
+
+// Wavefronts an atom (log2).  One wavefront alone works off its tiles at its
+// own latency, so few atoms leave the chip idle: four wavefronts an atom up to
+// two atoms a CU, two up to six, as long as each has a tile.  Forward +
+// backward us with 1 / 2 / 4 wavefronts an atom (Cu rows of 12 tiles): 500
+// atoms 75 / 48 / 41, 1,000 79 / 62 / 61, 1,500 103 / 81 / 80, 2,048 106 / 101 /
+// 110, 4,096 172 / 182 / 200; water rows of 8: 500 56 / 38 / 33, 1,000 59 / 48 /
+// 53, 1,500 75 / 65 / 71, 2,048 78 / 79 / 89.
+inline int split_of(int natoms, int nnei, int ncu) {
+  const int lp = natoms <= 2 * ncu ? 2 : natoms <= 6 * ncu ? 1 : 0;
+  return nnei > 32 ? lp : nnei > 16 && lp > 0 ? 1 : 0;
+}
 
 template <bool RESIDENT, class C>
 int launch2(bool fwd, void* out, const void* em, const void* gx, const int* atype,
             const void* image, const int* net_of, const int* ch_out, const Block2& bi, int nnets,
             int d3, int natoms, int nnei, hipStream_t st) {
-  const size_t lds = RESIDENT ? (size_t)nnets * (NET_BYTES + (fwd ? kBias4 : 0)) : 0;
-  // resident workgroups per device, cached per (device, direction, nnets)
+  // resident workgroups per device, cached per (device, direction, nnets, split)
   constexpr int kDev = 64, kRes = kResidentMaxBytes / NET_BYTES + 1;
-  static int cache[kDev][2][kRes];
-  int dev = 0;
+  static int cache[kDev][2][kRes][2];
+  int dev = 0, ncu = 0;
   DPK_HIP(hipGetDevice(&dev));
   DPK_REQUIRE(dev >= 0 && dev < kDev, DPK_ERR_ARG, "embed: device %d out of range", dev);
-  int& slots = cache[dev][fwd ? 0 : 1][RESIDENT ? nnets : 0];
+  DPK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  if (ncu < 1) ncu = 1;
+  const int lp = split_of(natoms, nnei, ncu);
+  const size_t lds = (RESIDENT ? (size_t)nnets * (NET_BYTES + (fwd ? kBias4 : 0)) : 0) +
+                     (fwd && lp > 0 ? kPartSums : 0);
+  int& slots = cache[dev][fwd ? 0 : 1][RESIDENT ? nnets : 0][lp > 0];
   if (slots == 0) {
-    int ncu = 0, per_cu = 0;
-    DPK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    int per_cu = 0;
     if (fwd)
       DPK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fwd2<RESIDENT, C>, 256, lds));
     else
       DPK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_bwd2<RESIDENT, C>, 256, lds));
-    slots = (ncu < 1 ? 1 : ncu) * (per_cu < 1 ? 1 : per_cu);
+    slots = ncu * (per_cu < 1 ? 1 : per_cu);
   }
-  const int groups = cdiv(natoms, 4);
+  const int groups = cdiv(natoms, 4 >> lp);
   const int pct = tune(DPK_TUNE_EMBED_GRID_PCT);
   const long want = pct == 0 ? groups : ((long)slots * pct + 99) / 100;
   const int grid = groups < want ? groups : (int)(want > 0 ? want : 1);
@@ -467,12 +515,12 @@ int launch2(bool fwd, void* out, const void* em, const void* gx, const int* atyp
   if (fwd)
     hipLaunchKernelGGL((k_fwd2<RESIDENT, C>), dim3(grid), dim3(256), lds, st,
                        static_cast<float*>(out), static_cast<const float*>(em), atype, img,
-                       net_of, ch_out, bi, nnets, d3, natoms, nnei);
+                       net_of, ch_out, bi, nnets, d3, natoms, nnei, lp);
   else
     hipLaunchKernelGGL((k_bwd2<RESIDENT, C>), dim3(grid), dim3(256), lds, st,
                        static_cast<float*>(out), static_cast<const float*>(em),
                        static_cast<const float*>(gx), atype, img, net_of, ch_out, bi, nnets, d3,
-                       natoms, nnei);
+                       natoms, nnei, lp);
   DPK_LAUNCHED();
   return DPK_OK;
 }

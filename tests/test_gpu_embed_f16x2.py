@@ -1,6 +1,7 @@
 """FP16X2 embedding kernels (csrc/embed_f16x2.hip) on their own, against the
 oracle's descriptor contraction and its autograd: resnet and time-step variants,
-nets in LDS and read from memory, block lengths around the 16-slot tile."""
+nets in LDS and read from memory, block lengths around the 16-slot tile, four,
+two and one wavefronts an atom (the limits are 512 and 1,536 atoms on 256 CUs)."""
 
 from types import SimpleNamespace
 
@@ -58,6 +59,11 @@ def _case(neuron, sel, one_side, natoms, dt, seed=5):
     ([10, 20, 40], [1, 31], True, 9, True),
     ([20, 30, 100], [40], True, 50, False),         # no doubling: no resnet
     ([20, 40, 100], [33], True, 4300, False),       # resnet of layer 2 only
+    ([25, 50, 100], [20, 33], True, 512, False),    # the last with four wavefronts an atom
+    ([25, 50, 100], [20, 33], False, 513, False),   # the first with two
+    ([25, 50, 100], [3, 30], True, 1536, True),     # the last with two
+    ([25, 50, 100], [3, 30], True, 1537, True),
+    ([25, 50, 100], [17], True, 100, False),        # two tiles: two wavefronts at most
     ([20, 50, 100], [15, 16, 17], False, 30, True),  # of layer 3 only, nine nets
 ])
 def test_embed_f16x2_vs_oracle(neuron, sel, one_side, natoms, dt):
