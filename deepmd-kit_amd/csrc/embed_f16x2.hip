@@ -470,6 +470,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
 constexpr int kResidentMaxBytes = 64 * 1024;
 constexpr int kPartSums = 4 * 8 * 16 * 16;  // forward, split atoms: four wavefronts' sums
 
+// Workgroups of a persistent grid per resident slot: with one, a slow XCD or a
+// ragged last round holds the launch; with eight, finished slots take what is
+// left, and a net is still copied to LDS once for several groups of atoms.
+// Forward + backward us with 1 / 4 / 8 a slot, or one a group: Cu (one net)
+// 8,788 atoms 356 / 333 / 331 / 332, 20,000 782 / 705 / 704 / 705, 131,072 5,227 /
+// 4,703 / 4,748 / 4,658; water (two nets) 8,788 275 / 275 / 276 / 274, 49,000 1,468 /
+// 1,418 / 1,399 / 1,435, 131,072 3,974 / 3,828 / 3,792 / 3,917.
+constexpr int kGridRounds = 8;
 
 // Wavefronts an atom (log2).  One wavefront alone works off its tiles at its
 // own latency, so few atoms leave the chip idle: four wavefronts an atom up to
@@ -509,7 +517,7 @@ int launch2(bool fwd, void* out, const void* em, const void* gx, const int* atyp
   }
   const int groups = cdiv(natoms, 4 >> lp);
   const int pct = tune(DPK_TUNE_EMBED_GRID_PCT);
-  const long want = pct == 0 ? groups : ((long)slots * pct + 99) / 100;
+  const long want = pct == 0 ? groups : ((long)kGridRounds * slots * pct + 99) / 100;
   const int grid = groups < want ? groups : (int)(want > 0 ? want : 1);
   const unsigned char* img = static_cast<const unsigned char*>(image);
   if (fwd)

@@ -57,7 +57,8 @@ enum {
   DPK_TUNE_NLIST_MODE = 0,      /* 0: staged cell neighbourhoods (default), 1: per-centre gather */
   DPK_TUNE_NLIST_STAGE_PCT = 1, /* staging capacity in % of the mean neighbourhood, 10..400 */
   DPK_TUNE_FORCE_MODE = 2,      /* 0: cell-blocked forces (default), 1: per-atom */
-  DPK_TUNE_EMBED_GRID_PCT = 3,  /* BF16 embedding persistent grid, % of resident slots;
+  DPK_TUNE_EMBED_GRID_PCT = 3,  /* 16-bit embedding persistent grid, % of the default (the
+                                   resident slots; eight times these for F16X2);
                                    0 = one workgroup per 4 atoms */
   DPK_TUNE_NLIST_WAVES = 4,     /* wavefronts per cell workgroup of the search: 0 = from the
                                    atoms per cell, else 4, 8 or 16 (rounded up) */
