@@ -24,7 +24,8 @@
 // Measured against tanh itself, all of G re-laid and every copy contracted:
 // 131,072 Cu atoms (12 tiles an atom) forward 2.47 -> 2.30 ms, backward 3.79 ->
 // 3.64; three wavefronts a SIMD for the backward without its 32 bytes of
-// scratch (outside the loop) 3.74, five for the forward 2.32.
+// scratch (outside the loop) 3.74, five for the forward 2.32 (all at one
+// workgroup per resident slot; kGridRounds takes the two to 1.79 and 2.96).
 // One wavefront an atom, or several where atoms are few (split_of), 16 slots a
 // tile; lane (g = lane / 16, c = lane % 16).
 #include "dpk_common.h"

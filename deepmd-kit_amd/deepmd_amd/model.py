@@ -11,6 +11,7 @@ hand-written adjoint kernels:
     embedding + R^T G      -> dpk_embed_fwd          (MFMA)
     G^T R R^T G            -> dpk_fit_descriptor_fwd (rows grouped by type)
     fitting net (+ grad)   -> hipBLASLt GEMMs + dpk_fit_layer_fwd / _bwd, dpk_fit_energy
+                              (FP64: dpk_fit_chain_f64; split FP16: dpk_fit_l1_*, dpk_fit_tail_*)
     dE/dxyz                -> dpk_fit_descriptor_bwd
     dE/d em (recompute)    -> dpk_embed_bwd          (MFMA)
     forces, virial         -> dpk_force_virial_cells + dpk_frame_sum
