@@ -6,13 +6,11 @@
 //
 // What bounds it: instruction issue.  A SIMD issues a plain VALU instruction
 // in 4 cycles, an exp2 / rcp in 8, a 16x16x32 MFMA in 8 (measured, the matrix
-// core itself being busy for 16); a tile of 16 slots costs 112 exp2 / rcp, 61
-// (forward) or 104 (backward) MFMAs and 240 or 456 others, of which the issue
+// core itself being busy for 16); a tile of 16 slots costs 112 exp2 / rcp, 60
+// (forward) or 104 (backward) MFMAs and 269 or 484 others, of which the issue
 // takes about 80% of the time.  What keeps the count down:
-//  * r = 1 / (1 + e^2x) stands for tanh x = 1 - 2 r: the sums over slots
-//    (forward) and channels (backward) run over r, the factor -2 and the sum
-//    of the other operand are applied once an atom or a tile, and
-//    1 - tanh^2 = 4 (r - r^2) is one FMA, its 4 applied once a tile;
+//  * with r = 1 / (1 + e^2x), 1 - tanh^2 x = 4 (r - r^2) is one FMA, its 4
+//    applied once a tile;
 //  * tangents carry constant factors (below) so that no operand is scaled
 //    before it is packed;
 //  * the forward's layer 3 has the slots on the rows (A = y2, B = W3^T), so
@@ -26,6 +24,16 @@
 // 3.64; three wavefronts a SIMD for the backward without its 32 bytes of
 // scratch (outside the loop) 3.74, five for the forward 2.32 (all at one
 // workgroup per resident slot; kGridRounds takes the two to 1.79 and 2.96).
+//
+// Precision.  The split operands are tanh, not r (whose 1/2 would cancel in the
+// sums; 32 FMAs a tile, 131,072 Cu atoms 7.77 -> 7.97 ms a step), and tangents
+// at one to two times their value (layers12); the resnet copies have an
+// accumulator of their own.  Errors against 64 bits, 2-norms, weights exact in
+// FP16 and scaled by 1 / 0.3 / 0.1 (nets of 32, 64, 128), r and quarter-scale
+// tangents -> now: xyz 1.1 / 1.5 / 2.0e-7 -> 1.0 / 1.3 / 1.6e-7, dE/d em 2.8 / 3.5
+// / 3.7e-7 -> 2.0 / 1.8 / 1.7e-7, its radial part 3.6 / 9.3 / 27e-7 -> 2.7 / 2.6 /
+// 4.1e-7; without resnets (20, 30, 100) at 0.1: 5.4e-7, 1.0e-6, 1.8e-4 -> 3.0e-7,
+// 3.0e-7, 2.2e-5.
 // One wavefront an atom, or several where atoms are few (split_of), 16 slots a
 // tile; lane (g = lane / 16, c = lane % 16).
 #include "dpk_common.h"
@@ -80,20 +88,29 @@ __device__ __forceinline__ v4u lds8(const unsigned char* p) {
 }
 
 constexpr v4f kZero4 = {0.f, 0.f, 0.f, 0.f};
-constexpr unsigned kOne2 = 0x3c003c00u;  // two FP16 ones
 
 // Forward only: the layer-3 bias of channel c four times over, after the net
 // image in LDS (one 16-byte read starts a lane's accumulator).
 constexpr int kBias4 = P3 * 16;
 
-// Resident nets: copied to LDS once per (persistent) workgroup.
-template <bool BIAS4>
+// Resident nets: copied to LDS once per (persistent) workgroup, w1 (which only
+// the tangents use) as S1 w1.
+template <bool BIAS4, int S1>
 __device__ __forceinline__ void stage(unsigned char* dst, const unsigned char* src, int nnets) {
   constexpr int kOut = NET_BYTES + (BIAS4 ? kBias4 : 0);
   for (int k = 0; k < nnets; ++k) {
     const int4* s4 = reinterpret_cast<const int4*>(src + (size_t)k * NET_BYTES);
     int4* d4 = reinterpret_cast<int4*>(dst + k * kOut);
-    for (int q = threadIdx.x; q < NET_BYTES / 16; q += blockDim.x) d4[q] = s4[q];
+    for (int q = threadIdx.x; q < NET_BYTES / 16; q += blockDim.x) {
+      int4 v = s4[q];
+      if (S1 != 1 && q < (V_W1 + P1) / 4) {
+        v.x = __float_as_int(S1 * __int_as_float(v.x));
+        v.y = __float_as_int(S1 * __int_as_float(v.y));
+        v.z = __float_as_int(S1 * __int_as_float(v.z));
+        v.w = __float_as_int(S1 * __int_as_float(v.w));
+      }
+      d4[q] = v;
+    }
     if constexpr (BIAS4) {
       const float* b = reinterpret_cast<const float*>(src + (size_t)k * NET_BYTES) + V_B3K;
       float* o = reinterpret_cast<float*>(dst + k * kOut + NET_BYTES);
@@ -104,11 +121,14 @@ __device__ __forceinline__ void stage(unsigned char* dst, const unsigned char* s
 }
 
 // Layers 1-2 for the lane's slot (channels 16 m + 4 g + i): y2 and, for the
-// backward, t2 = (dy2/ds) K / 16.  With K = 2 log2 e the image's weights are
-// K W; t1 = w1 (r - r^2) = dy1/ds / 4 goes through them as it is, and
-// K W t1 (r2 - r2^2) = (K / 16) (dy2/ds without the resnet), to which the
-// resnet adds (K / 4) t1.
-template <bool TANGENT, class C>
+// backward, t2 = (dy2/ds) K / 2.  With K = 2 log2 e the image's weights are
+// K W; t1 = 8 w1 (r - r^2) = 2 dy1/ds goes through them as it is, and
+// K W t1 (r2 - r2^2) = (K / 2) (dy2/ds without the resnet), to which the
+// resnet adds (K / 4) t1.  The factor 2 of t1 sets the scale at which all
+// tangents are split: 2, 1.4 and (k_bwd2) 1.04 of the derivatives, so that
+// their low parts stay out of FP16's subnormals as far as those of the values
+// do and no derivative below 62,900 overflows.  SCALED: w1 is 8 w1 already.
+template <bool TANGENT, bool SCALED, class C>
 __device__ __forceinline__ void layers12(const unsigned char* nb, float s, int g, int c,
                                          float y2[4][4], float t2[4][4]) {
   constexpr bool FOLD = C::RES2 == 2 && !C::IDT;  // y2 = (1 + y1) - 2 r2
@@ -122,7 +142,8 @@ __device__ __forceinline__ void layers12(const unsigned char* nb, float s, int g
       const float r = tanh_r(__builtin_fmaf(s, vec[V_W1K + ch], vec[V_B1K + ch]));
       y1[m][i] = __builtin_fmaf(-2.0f, r, 1.0f);
       if (FOLD) e1[m][i] = __builtin_fmaf(-2.0f, r, 2.0f);
-      if (TANGENT) t1[m][i] = __builtin_fmaf(-r, r, r) * vec[V_W1 + ch];
+      if (TANGENT)
+        t1[m][i] = __builtin_fmaf(-r, r, r) * (SCALED ? vec[V_W1 + ch] : 8.0f * vec[V_W1 + ch]);
     }
   const v4u B1 = pack8(y1[0], y1[1]), B1l = lo8(y1[0], y1[1], B1);
   v4u T1, T1l;
@@ -164,11 +185,10 @@ __device__ __forceinline__ void layers12(const unsigned char* nb, float s, int g
   }
 }
 
-// r (or, with time steps, -idt tanh / 2) of a layer-3 argument
+// tanh (with time steps: idt tanh) from r; idt2 = -2 idt
 template <class C>
-__device__ __forceinline__ float r3(float u, float idt) {
-  const float r = tanh_r(u);
-  return C::IDT ? __builtin_fmaf(r, idt, -0.5f * idt) : r;
+__device__ __forceinline__ float tanh3(float r, float idt, float idt2) {
+  return C::IDT ? __builtin_fmaf(r, idt2, idt) : __builtin_fmaf(-2.0f, r, 1.0f);
 }
 
 template <bool RESIDENT, class C>
@@ -179,7 +199,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
   extern __shared__ __align__(16) unsigned char lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-  if (RESIDENT) stage<true>(lds, nets, nnets);
+  if (RESIDENT) stage<true, 1>(lds, nets, nnets);
   const float id[4] = {c == 4 * g ? 1.f : 0.f, c == 4 * g + 1 ? 1.f : 0.f,
                        c == 4 * g + 2 ? 1.f : 0.f, c == 4 * g + 3 ? 1.f : 0.f};
   const v2u ident = pack4(id);
@@ -191,9 +211,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
     int ti = valid ? atype[atom] : 0;
     ti = ti < 0 ? 0 : ti;
     const float* e = em + (size_t)(valid ? atom : 0) * nnei * 4;
-    // xyz nnei = accS + accY - 2 acc: sums over slots of R, R y2 and R r3.
-    // Rows 0-3 are R's hi parts, rows 4-7 its lo parts (added once an atom).
-    v4f acc[8], accY[4], accS = kZero4;
+    // xyz nnei = accY + acc: sums over slots of R y2 and R tanh.  Rows 0-3 are
+    // R's hi parts, rows 4-7 its lo parts (added once an atom).
+    v4f acc[8], accY[4];
 #pragma unroll
     for (int m = 0; m < 8; ++m) acc[m] = kZero4;
 #pragma unroll
@@ -214,7 +234,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
 #pragma unroll
           for (int m = 0; m < 8; ++m)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[m][i] -= 0.5f * pt[i * P3 + 16 * m + c];
+            for (int i = 0; i < 4; ++i) acc[m][i] += pt[i * P3 + 16 * m + c];
         }
       }
       const int first = (part - tix) & ((1 << lp) - 1);
@@ -236,10 +256,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
         if (c >= 4) rT = rl;
         const v4u RT = {rT[0], rT[1], rT[0], rT[1]};  // against (hi, lo) of the same slots
         float y2[4][4], t2[4][4];
-        layers12<false, C>(nb, s, g, c, y2, t2);
+        layers12<false, false, C>(nb, s, g, c, y2, t2);
         const v4u B2[2] = {pack8(y2[0], y2[1]), pack8(y2[2], y2[3])};
         const v4u B2l[2] = {lo8(y2[0], y2[1], B2[0]), lo8(y2[2], y2[3], B2[1])};
-        if constexpr (!C::IDT) accS = E::mfma16(rT, v2u{kOne2, kOne2}, accS);
         if constexpr (C::RES3 == 2) {
 #pragma unroll
           for (int m = 0; m < 4; ++m) {
@@ -266,10 +285,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
           u = E::mfma32(B2[1], a1, u);
           u = E::mfma32(B2l[0], a0, u);
           u = E::mfma32(B2l[1], a1, u);  // row 4 g + i = slot, column c = channel
-          const float idt = C::IDT ? vec[V_IDT3 + 16 * m + c] : 1.0f;
+          const float idt = C::IDT ? vec[V_IDT3 + 16 * m + c] : 1.0f, idt2 = -2.0f * idt;
           float v[4];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) v[i] = r3<C>(u[i], idt);
+          for (int i = 0; i < 4; ++i) v[i] = tanh3<C>(tanh_r(u[i]), idt, idt2);
           const v2u vh = pack4(v), vl = lo4(v, vh);
           acc[m] = E::mfma32(RT, v4u{vh[0], vh[1], vl[0], vl[1]}, acc[m]);
           __builtin_amdgcn_sched_barrier(0);
@@ -281,7 +300,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
     for (int m = 0; m < 8; ++m)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        float v = __builtin_fmaf(-2.0f, acc[m][i], accS[i] + accY[m & 3][i]);
+        const float v = acc[m][i] + accY[m & 3][i];
         acc[m][i] = v + __shfl_xor(v, 16, 64);
       }
     if (lp > 0) {  // the other wavefronts' sums, in their order
@@ -319,7 +338,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
   extern __shared__ __align__(16) unsigned char lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-  if (RESIDENT) stage<false>(lds, nets, nnets);
+  if (RESIDENT) stage<false, 8>(lds, nets, nnets);
   // 1 << lp wavefronts an atom, each with every (1 << lp)-th tile
   const int apw = 4 >> lp, part = wave & ((1 << lp) - 1);
   for (int base = blockIdx.x * apw; base < natoms; base += gridDim.x * apw) {
@@ -348,7 +367,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
     const int comp = c & 3;
     v4u gxa[4], gxc[2];  // gxc: summed over the channels of one resnet copy
     float cl[2][4], ch[2][4];
-    v4f S = kZero4;  // sum over channels of gx (tanh = 1 - 2 r)
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
       float lo[4], hi[4];
@@ -377,7 +395,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
           if (c >= 4) gxc[k] = l2;
         }
       }
-      if constexpr (!C::IDT) S = E::mfma32(gxa[p], v4u{kOne2, kOne2, kOne2, kOne2}, S);
     }
     int tix = 0;  // tiles of the blocks before this one
     for (int t = 0; t < bi.ntypes; ++t) {
@@ -399,26 +416,25 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
         const int slot = s0 + c;
         const float s = slot < b1 ? e[slot * 4] : 0.f;
         float y2[4][4], t2[4][4];
-        layers12<true, C>(nb, s, g, c, y2, t2);
+        layers12<true, RESIDENT, C>(nb, s, g, c, y2, t2);
         const v4u B2[2] = {pack8(y2[0], y2[1]), pack8(y2[2], y2[3])};
         const v4u B2l[2] = {lo8(y2[0], y2[1], B2[0]), lo8(y2[2], y2[3], B2[1])};
         const v4u T2[2] = {pack8(t2[0], t2[1]), pack8(t2[2], t2[3])};
         const v4u T2l[2] = {lo8(t2[0], t2[1], T2[0]), lo8(t2[2], t2[3], T2[1])};
-        // dR[comp][slot c] = S + gx y2 - 2 gx r3, kept over -2;
-        // dE/ds = sum_comp R[comp] (64 / K^2) Mx[comp], Mx = gx (K W3 t2) (r3 - r3^2)
+        // dR[comp][slot c] = gx y2 + gx tanh;
+        // dE/ds = sum_comp R[comp] (8 / K^2) Mx[comp], Mx = gx (K W3 t2) (r3 - r3^2)
         //         + (K / 4) gx t2 (the resnet copies)
-        v4f dR = S, Mx = kZero4;
+        v4f dR = kZero4, Mx = kZero4, dRc = kZero4;
         if constexpr (C::RES3 == 2) {
 #pragma unroll
           for (int p = 0; p < 2; ++p) {
-            dR = E::mfma32(gxc[p], B2[p], dR);
+            dRc = E::mfma32(gxc[p], B2[p], dRc);
             Mx = E::mfma32(gxc[p], T2[p], Mx);
-            dR = E::mfma32(gxc[p], B2l[p], dR);
+            dRc = E::mfma32(gxc[p], B2l[p], dRc);
             Mx = E::mfma32(gxc[p], T2l[p], Mx);
           }
           Mx *= K2L2E / 4;
         }
-        dR *= -0.5f;
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
           float v[2][4], dv[2][4];
@@ -439,7 +455,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
             for (int i = 0; i < 4; ++i) {
               const float idt = C::IDT ? vec[V_IDT3 + 16 * m + 4 * g + i] : 1.0f;
               const float r = tanh_r(u[i]);
-              v[h][i] = C::IDT ? __builtin_fmaf(r, idt, -0.5f * idt) : r;
+              v[h][i] = tanh3<C>(r, idt, -2.0f * idt);
               const float d = __builtin_fmaf(-r, r, r) * tu[i];
               dv[h][i] = C::IDT ? d * idt : d;
             }
@@ -451,15 +467,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
           Mx = E::mfma32(gxa[p], lo8(dv[0], dv[1], dh), Mx);
           __builtin_amdgcn_sched_barrier(0);
         }
+        dR += dRc;
         // lanes g = 1 hold rows 4-7 (the gx_lo products): fold them into ds
         // and dR of the lanes g = 0 (the components are the same)
         float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
         if (g < 2 && slot < b1) r = *reinterpret_cast<const float4*>(e + slot * 4);
-        float ds = (64.0f / (K2L2E * K2L2E)) *
+        float ds = (8.0f / (K2L2E * K2L2E)) *
                    (r.x * Mx[0] + r.y * Mx[1] + r.z * Mx[2] + r.w * Mx[3]);
         ds += __shfl_xor(ds, 16, 64);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) dR[i] = -2.0f * (dR[i] + __shfl_xor(dR[i], 16, 64));
+        for (int i = 0; i < 4; ++i) dR[i] += __shfl_xor(dR[i], 16, 64);
         if (g == 0 && slot < b1)
           *reinterpret_cast<float4*>(nd + slot * 4) =
               make_float4((dR[0] + ds) * unq, dR[1] * unq, dR[2] * unq, dR[3] * unq);

@@ -17,9 +17,9 @@ DEV = "cuda"
 
 # The weights are FP16 values (below), so what is left is the split operands'
 # 2^-22 and FP32's tanh (1e-7), grown by a factor of about two a layer, and FP32
-# sums of up to 200 slots: below 1e-5 of the largest value; a lost low part
-# would be 2^-11 = 5e-4.
-TOL = 2e-5
+# sums of up to 200 slots, whose errors average out: below 2e-6 of the largest
+# value; a lost low part would be 2^-11 = 5e-4.
+TOL = 2e-6
 K = 2.8853900817779268  # the kernels' weights are rounded after this scaling
 
 
@@ -87,3 +87,63 @@ def test_embed_f16x2_vs_oracle(neuron, sel, one_side, natoms, dt):
         err = np.max(np.abs(got.cpu().numpy() - ref)) / np.max(np.abs(ref))
         print(f"{what} {neuron} {sel} n={natoms}: {err:.2e}", flush=True)
         assert err < TOL, what
+
+
+# Rounding at the scale of the operands: with weights that are FP16 values and
+# tangents split at one to two times the derivatives themselves, a value or a
+# tangent keeps 2^-22 of itself and at worst 2^-25 absolute (FP16's subnormals);
+# the second decides where weights are small and no resnet copy holds the
+# derivatives up.  2-norms of the error over the result's: (xyz, net_deriv, ds),
+# a third above what kernels that split tanh and the tangents at this scale
+# reach on these cases.
+SMALL = {
+    ((32, 64, 128), 1.0): (2.2e-7, 3.1e-7, 3.8e-7),
+    ((32, 64, 128), 0.3): (2.2e-7, 3.1e-7, 5.0e-7),
+    ((32, 64, 128), 0.1): (2.4e-7, 3.1e-7, 1.3e-6),
+    ((20, 30, 100), 1.0): (2.2e-7, 3.3e-7, 4.2e-7),
+    ((20, 30, 100), 0.3): (3.6e-7, 4.0e-7, 1.6e-6),
+    ((20, 30, 100), 0.1): (4.0e-7, 4.1e-7, 3.2e-5),
+    ((20, 40, 100), 0.1): (3.6e-7, 4.0e-7, 2.8e-6),
+    ((20, 50, 100), 0.1): (3.6e-7, 4.8e-7, 9.6e-6),
+}
+
+
+@pytest.mark.parametrize("neuron,scale", list(SMALL))
+@pytest.mark.parametrize("natoms", [64, 1600])
+def test_embed_f16x2_operand_bits(neuron, scale, natoms):
+    """Errors of the split operands alone, also for small weights, and of the
+    radial derivative ds apart from dE/dR (gx without its first component)."""
+    d, at, em, nl, gx = _case(list(neuron), [60], True, natoms, False)
+    rng = np.random.default_rng(9)
+    de = d["model"]["descriptor"]
+    de["@variables"]["davg"]["value"] = np.zeros((1, 60, 4)).tolist()
+    for net in de["embeddings"]["networks"]:
+        for k, ly in enumerate(net["layers"]):
+            w = ly["@variables"]["w"]
+            v = np.asarray(w["value"]) * scale
+            v = (v * K).astype(np.float16).astype(np.float64) / K if k else v.astype(np.float32)
+            w["value"] = np.asarray(v, np.float64).tolist()
+    em = rng.normal(size=em.shape).astype(np.float32)
+    nl = np.zeros_like(nl)
+    om = sea.model_from_serialized(d)
+    m = SeAModel(d, "f16x2", DEV)
+    to = lambda a: torch.tensor(a, device=DEV).contiguous()  # noqa: E731
+    err = []
+    for first in (1.0, 0.0):
+        gx = gx.copy()
+        gx[:, 0] *= first
+        e = torch.tensor(em, dtype=torch.float64, requires_grad=True)
+        _, xyz = sea.descriptor_from_env(om, e, torch.tensor(at).long(),
+                                         torch.ones(em.shape[:2], dtype=torch.int32))
+        nd, = torch.autograd.grad((xyz * torch.tensor(gx)).sum(), e)
+        s = SimpleNamespace(fs=SimpleNamespace(natoms=natoms), em=to(em), atype=to(at),
+                            nlist=to(nl), gxyz=to(gx), nd=torch.zeros(*em.shape, device=DEV),
+                            xyz=torch.zeros(natoms, 4, m.d3, device=DEV))
+        st = torch.cuda.current_stream().cuda_stream
+        m._embed_forward(s, st)
+        m._embed_backward(s, st)
+        torch.cuda.synchronize()
+        pairs = ((s.xyz, xyz.detach()), (s.nd, nd)) if first else ((s.nd[..., 0], nd[..., 0]),)
+        err += [float((g.cpu().double() - r).norm() / r.norm()) for g, r in pairs]
+    print(f"{neuron} x {scale} n={natoms}: " + " ".join(f"{v:.2e}" for v in err), flush=True)
+    assert all(v < t for v, t in zip(err, SMALL[neuron, scale])), err
