@@ -29,12 +29,21 @@
 // slots 4 i + g, channel c -- is the operand the contraction needs; only y2
 // (the resnet copy of layer 3) is turned through LDS for it.
 //
-// The workgroup holds every net's weights in LDS in fragment order (one
-// conflict-free 8-byte read a lane and MFMA) when they fit, else lanes read
-// them from memory through the caches.  Workgroups are persistent (one a CU);
-// `split` wavefronts share an atom, taking every split-th tile of it and
-// adding their parts in LDS in a fixed order, so that a few hundred atoms
-// fill the chip as well as many thousands.
+// The workgroup holds the weights in LDS in fragment order (one conflict-free
+// 8-byte read a lane and MFMA): of every net where they fit together (one of
+// width 128, two of 100), else a group of nets at a time, the atoms that use it
+// dealt to the wavefronts (k_fwd64 / k_bwd64, ALL false).  Workgroups are
+// persistent (one a CU); `split` wavefronts share an atom, taking every
+// split-th tile of it and adding their parts in LDS in a fixed order, so that
+// a few hundred atoms fill the chip as well as many thousands.
+//
+// Groups, against fragments read from memory through the caches (activations
+// spilled: 900 to 1,500 bytes a lane), forward / backward us: two nets of 128,
+// water of 375 atoms 154 / 178 -> 73 / 104, 1,536 482 / 577 -> 152 / 233, 5,184
+// 1,352 / 1,593 -> 380 / 581; four nets of 100: 81 atoms 34 / 42 -> 34 / 48, 375
+// 62 / 75 -> 70 / 91, 1,536 210 / 236 -> 136 / 196, 5,184 580 / 643 -> 327 / 473;
+// sixteen of 128, 14,374 atoms of four types: 3,990 / 5,224 -> 1,096 / 1,720;
+// gelu, two nets of 100, 1,536 atoms 728 / 888 -> 416 / 528.
 //
 // Measured (forward / backward, us), against one wavefront an atom, every
 // slot, 16 x 16 contractions and the library exp: water of 81 atoms 285 / 292
@@ -66,6 +75,7 @@ struct EmbArgs {
   const double* pad;     // may be null
   double* out;
   int ntypes, nnets, d3, natoms, nnei, split;
+  int room;              // nets that fit in LDS together
   int res2, res3, idt;   // general kernels only
   ActSpec act;
   int sec[kMaxTypes + 1];
@@ -96,12 +106,13 @@ __device__ __forceinline__ void wave_sync() {
 
 // Channel steps: S1 of layer 1, 2 S1 of layer 2, 4 S1 of layer 3; step t,
 // channel 4 t + g.  Internal (packed) channel of step t: 32 (t / S1) + 4 (t %
-// S1) + g.  G (general): S1 = 8, run-time resnet modes, time steps and
-// activation; otherwise tanh, doubling resnets, no time steps.
-template <int S1_, bool G_>
+// S1) + g.  Kinds: tanh with doubling resnets and no time steps; G (general, S1
+// = 8): run-time resnet modes and time steps, with tanh or any activation.
+enum { kPlain = 0, kTanh = 1, kAny = 2 };
+template <int S1_, int KIND_>
 struct Shape {
-  static constexpr int S1 = S1_;
-  static constexpr bool G = G_;
+  static constexpr int S1 = S1_, KIND = KIND_;
+  static constexpr bool G = KIND != kPlain;
   static constexpr int S2 = 2 * S1, S3 = 4 * S1;
   static constexpr int B2 = (S2 + 3) / 4, B3 = S1;  // 16-channel blocks
   // one net in LDS, in doubles
@@ -115,95 +126,179 @@ struct Shape {
   }
 };
 
-// Parameters of a net, from LDS (fragment order) or from memory.
-template <class SH, bool LDS>
+// Parameters of a net in LDS.
+template <class SH>
 struct Net {
   const double* p;
   int lane;
   // between 16-channel blocks: the next block's weights are not read (and held
   // in registers) early
-  __device__ __forceinline__ void fence() const {
-    if constexpr (!LDS) asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-  }
+  __device__ __forceinline__ void fence() const { __builtin_amdgcn_sched_barrier(0); }
   __device__ __forceinline__ double w2(int m, int ks) const {
-    if constexpr (LDS) return p[SH::oW2 + (m * SH::S1 + ks) * 64 + lane];
-    const int n = 16 * m + (lane & 15);
-    if (n >= 4 * SH::S2) return 0.0;
-    return p[O_W2 + SH::inner(n) * P1 + 4 * ks + (lane >> 4)];
+    return p[SH::oW2 + (m * SH::S1 + ks) * 64 + lane];
   }
   __device__ __forceinline__ double w3(int m, int ks) const {
-    if constexpr (LDS) return p[SH::oW3 + (m * SH::S2 + ks) * 64 + lane];
-    return p[O_W3 + SH::inner(16 * m + (lane & 15)) * P2 + 32 * (ks / SH::S1) +
-             4 * (ks % SH::S1) + (lane >> 4)];
+    return p[SH::oW3 + (m * SH::S2 + ks) * 64 + lane];
   }
-  __device__ __forceinline__ double w1(int n) const { return p[LDS ? SH::vW1 + n : n]; }
-  __device__ __forceinline__ double b1(int n) const { return p[LDS ? SH::vB1 + n : O_B1 + n]; }
-  __device__ __forceinline__ double b2(int n) const {
-    return LDS ? p[SH::vB2 + n] : (n < 4 * SH::S2 ? p[O_B2 + SH::inner(n)] : 0.0);
-  }
-  __device__ __forceinline__ double b3(int n) const {
-    return p[LDS ? SH::vB3 + n : O_B3 + SH::inner(n)];
-  }
-  __device__ __forceinline__ double i2(int n) const {
-    return p[LDS ? SH::vI2 + n : O_I2 + SH::inner(n)];
-  }
-  __device__ __forceinline__ double i3(int n) const {
-    return p[LDS ? SH::vI3 + n : O_I3 + SH::inner(n)];
-  }
+  __device__ __forceinline__ double w1(int n) const { return p[SH::vW1 + n]; }
+  __device__ __forceinline__ double b1(int n) const { return p[SH::vB1 + n]; }
+  __device__ __forceinline__ double b2(int n) const { return p[SH::vB2 + n]; }
+  __device__ __forceinline__ double b3(int n) const { return p[SH::vB3 + n]; }
+  __device__ __forceinline__ double i2(int n) const { return p[SH::vI2 + n]; }
+  __device__ __forceinline__ double i3(int n) const { return p[SH::vI3 + n]; }
 };
 
-template <class SH>
-__device__ __forceinline__ void stage_nets(double* w, const double* params, int nnets) {
-  for (int k = 0; k < nnets; ++k) {
-    double* o = w + (size_t)k * SH::size;
+// Nets list[p0 .. p1) (list null: nets p0 .. p1) to LDS in fragment order, a
+// fragment (64 values) a wavefront and load, all of a wavefront's loads of a
+// net in flight together.
+template <class SH, int NW>
+__device__ __forceinline__ void stage_nets(double* w, const double* params,
+                                           const unsigned short* list, int p0, int p1, int wave,
+                                           int lane) {
+  constexpr int F2 = SH::B2 * SH::S1, F3 = SH::B3 * SH::S2;
+  const int g = lane >> 4, c = lane & 15;
+  for (int q = p0; q < p1; ++q) {
+    const int k = list != nullptr ? __builtin_amdgcn_readfirstlane(list[q]) : q;
+    double* o = w + (size_t)(q - p0) * SH::size;
     const double* p = params + (size_t)k * NET;
-    for (int q = threadIdx.x; q < SH::size; q += blockDim.x) {
+#pragma unroll
+    for (int i = 0; i < (F2 + NW - 1) / NW; ++i) {
+      const int f = wave + NW * i, n = 16 * (f / SH::S1) + c;
+      if (f < F2)
+        o[SH::oW2 + f * 64 + lane] =
+            n < 4 * SH::S2 ? p[O_W2 + SH::inner(n) * P1 + 4 * (f % SH::S1) + g] : 0.0;
+    }
+#pragma unroll
+    for (int i = 0; i < (F3 + NW - 1) / NW; ++i) {
+      const int f = wave + NW * i;
+      if (f < F3)
+        o[SH::oW3 + f * 64 + lane] = p[O_W3 + SH::inner(16 * (f / SH::S2) + c) * P2 +
+                                       SH::inner(4 * (f % SH::S2) + g)];
+    }
+    for (int i = SH::oV + threadIdx.x; i < SH::size; i += 64 * NW) {
       double v = 0.0;
-      if (q < SH::oW3) {
-        const int l = q & 63, ks = (q >> 6) % SH::S1, n = 16 * ((q >> 6) / SH::S1) + (l & 15);
-        if (n < 4 * SH::S2) v = p[O_W2 + SH::inner(n) * P1 + 4 * ks + (l >> 4)];
-      } else if (q < SH::oV) {
-        const int r = q - SH::oW3, l = r & 63, ks = (r >> 6) % SH::S2;
-        const int n = 16 * ((r >> 6) / SH::S2) + (l & 15);
-        v = p[O_W3 + SH::inner(n) * P2 + SH::inner(4 * ks + (l >> 4))];
-      } else if (q < SH::vB1) {
-        v = p[q - SH::vW1];
-      } else if (q < SH::vB2) {
-        v = p[O_B1 + q - SH::vB1];
-      } else if (q < SH::vB3) {
-        if (q - SH::vB2 < 4 * SH::S2) v = p[O_B2 + SH::inner(q - SH::vB2)];
-      } else if (q < SH::vI2) {
-        v = p[O_B3 + SH::inner(q - SH::vB3)];
-      } else if (q < SH::vI3) {
-        if (q - SH::vI2 < 4 * SH::S2) v = p[O_I2 + SH::inner(q - SH::vI2)];
+      if (i < SH::vB1) {
+        v = p[i - SH::vW1];
+      } else if (i < SH::vB2) {
+        v = p[O_B1 + i - SH::vB1];
+      } else if (i < SH::vB3) {
+        if (i - SH::vB2 < 4 * SH::S2) v = p[O_B2 + SH::inner(i - SH::vB2)];
+      } else if (i < SH::vI2) {
+        v = p[O_B3 + SH::inner(i - SH::vB3)];
+      } else if (i < SH::vI3) {
+        if (i - SH::vI2 < 4 * SH::S2) v = p[O_I2 + SH::inner(i - SH::vI2)];
       } else {
-        v = p[O_I3 + SH::inner(q - SH::vI3)];
+        v = p[O_I3 + SH::inner(i - SH::vI3)];
       }
-      o[q] = v;
+      o[i] = v;
     }
   }
+}
+
+// Nets that don't fit in LDS together are taken in groups of `room`: a
+// workgroup lists the nets that its atoms use, stages a group, works off the
+// type blocks that use one of its nets, and goes on to the next.
+constexpr int kMaxNets = kMaxTypes * kMaxTypes;
+struct Groups {
+  unsigned short list[kMaxNets];  // the nets used, ascending
+  unsigned short at[kMaxNets];    // a net's place in the list (kMaxNets: not used)
+  unsigned types;                 // the types of the atoms, a bit each
+};
+
+// Lists the nets of the workgroup's atoms, `per` of them a turn of the grid
+// (virtual atoms count as type 0), and returns how many there are.
+__device__ __forceinline__ int list_nets(const EmbArgs& A, Groups& G, int per) {
+  if (threadIdx.x == 0) G.types = 0;
+  for (int q = threadIdx.x; q < kMaxNets; q += blockDim.x) G.at[q] = kMaxNets;
+  __syncthreads();
+  unsigned m = 0;
+  for (int q = threadIdx.x;; q += blockDim.x) {
+    const long base = ((long)blockIdx.x + (long)(q / per) * gridDim.x) * per;
+    if (base >= A.natoms) break;
+    const long atom = base + q % per;
+    if (atom < A.natoms) m |= 1u << (A.atype[atom] < 0 ? 0 : A.atype[atom]);
+  }
+  if (m != 0) atomicOr(&G.types, m);
+  __syncthreads();
+  for (int q = threadIdx.x; q < A.ntypes * A.ntypes; q += blockDim.x) {
+    const int t = q % A.ntypes;
+    if ((G.types >> (q / A.ntypes) & 1) && A.sec[t + 1] > A.sec[t]) G.at[A.net_of[q]] = 0;
+  }
+  __syncthreads();
+  int n = 0;
+  for (int k = 0; k < A.nnets; ++k) {  // (every thread counts)
+    const bool use = G.at[k] < kMaxNets;
+    if (use && threadIdx.x == 0) G.list[n] = (unsigned short)k;
+    n += use;
+  }
+  __syncthreads();
+  for (int q = threadIdx.x; q < n; q += blockDim.x) G.at[G.list[q]] = (unsigned short)q;
+  __syncthreads();
+  return n;
+}
+
+// The blocks (a bit each) of centre type ti that use a net of the group [p0,
+// p1); earlier: whether a former group had one.
+__device__ __forceinline__ unsigned group_blocks(const EmbArgs& A, const Groups& G, int p0, int p1,
+                                                 int ti, bool& earlier) {
+  unsigned m = 0;
+  earlier = false;
+  for (int t = 0; t < A.ntypes; ++t) {
+    if (A.sec[t + 1] <= A.sec[t]) continue;
+    const int at = __builtin_amdgcn_readfirstlane(G.at[A.net_of[ti * A.ntypes + t]]);
+    earlier = earlier || at < p0;
+    if (at >= p0 && at < p1) m |= 1u << t;
+  }
+  return m;
+}
+
+// The centre types (a bit each) that have a block in the group.
+__device__ __forceinline__ unsigned group_types(const EmbArgs& A, const Groups& G, int p0, int p1,
+                                                int lane) {
+  bool has = false;
+  if (lane < A.ntypes)
+    for (int t = 0; t < A.ntypes; ++t) {
+      const int at = G.at[A.net_of[lane * A.ntypes + t]];
+      has = has || (A.sec[t + 1] > A.sec[t] && at >= p0 && at < p1);
+    }
+  return (unsigned)__ballot(has);
+}
+
+// Of the workgroup's atoms q0 .. q0 + 63 (`per` of them a turn of the grid)
+// those of the given types, a bit each; first: atom of the bit 0, or past the
+// end.
+__device__ __forceinline__ int atom_at(int q, int per) {
+  return (int)((blockIdx.x + (long)(q / per) * gridDim.x) * per + q % per);
+}
+__device__ __forceinline__ unsigned long long atoms_of(const EmbArgs& A, unsigned types, int q0,
+                                                       int per, int lane) {
+  const int atom = atom_at(q0 + lane, per);
+  bool take = false;
+  if (atom < A.natoms) take = types >> (A.atype[atom] < 0 ? 0 : A.atype[atom]) & 1;
+  return __ballot(take);
+}
+__device__ __forceinline__ int nth_bit(unsigned long long m, int n) {
+  for (; n > 0; --n) m &= m - 1;
+  return __ffsll(m) - 1;
 }
 
 // activation f and (DERIV) its derivative d at z
 template <class SH, bool DERIV>
 __device__ __forceinline__ void act64(const EmbArgs& A, const double* tab, double z, double& f,
                                       double& d) {
-  if constexpr (SH::G) {
-    if (A.act.id != DPK_ACT_TANH) {
-      const Act2 r = act_general(A.act, z);
-      f = r.f;
-      d = r.d;
-      return;
-    }
+  if constexpr (SH::KIND == kAny) {
+    const Act2 r = act_general(A.act, z);
+    f = r.f;
+    d = r.d;
+    return;
   }
   f = tanh64(z, tab);
   if constexpr (DERIV) d = __fma_rn(-f, f, 1.0);
 }
 
 // Layers 1 and 2 for the lane's slot (s), with the tangents d/ds (DERIV).
-template <class SH, bool LDS, bool DERIV>
-__device__ __forceinline__ void layers12(const EmbArgs& A, const Net<SH, LDS>& net,
+template <class SH, bool DERIV>
+__device__ __forceinline__ void layers12(const EmbArgs& A, const Net<SH>& net,
                                          const double* tab, double s, int g, double (&y2)[SH::S2],
                                          double (&d2)[DERIV ? SH::S2 : 1]) {
   double y1[SH::S1], d1[DERIV ? SH::S1 : 1];
@@ -262,16 +357,16 @@ __device__ __forceinline__ bool same_rows(const double* em, int b, int e, int la
 }
 
 // Walks the tiles (16 slots from s0, up to b1) of an atom that fall to
-// wavefront `sub` of `split`.  Forward: a block ends at its last real
-// neighbour.  Backward (BWD): the padding rows after it are one slot more
+// wavefront `sub` of `split`, in the blocks of the mask.  Forward: a block ends
+// at its last real neighbour.  Backward (BWD): the padding rows after it are one slot more
 // where they are all the same (fold), for all of which that slot stands;
 // else they are computed like any other.
 template <bool BWD, class F>
-__device__ __forceinline__ void for_tiles(const EmbArgs& A, int atom, int sub, int lane,
-                                          F&& body) {
+__device__ __forceinline__ void for_tiles(const EmbArgs& A, int atom, int ti, unsigned blocks,
+                                          int sub, int lane, F&& body) {
   int turn = sub;  // tiles until this wavefront's next one
-  const int ti = A.atype[atom] < 0 ? 0 : A.atype[atom];
   for (int t = 0; t < A.ntypes; ++t) {
+    if (!(blocks >> t & 1)) continue;
     const int b0 = A.sec[t];
     int b1 = A.sec[t + 1];
     const int end = b1;
@@ -296,15 +391,19 @@ __device__ __forceinline__ void for_tiles(const EmbArgs& A, int atom, int sub, i
 template <class SH>
 constexpr int kFwdScratch = (4 * 16 * SH::B3 > 16 * 17 ? 4 * 16 * SH::B3 : 16 * 17);
 
-template <class SH, bool LDS, int NW>
+// A workgroup's LDS, in doubles: the table and (nets in groups) their list, the
+// scratch, the nets.
+constexpr int kHeadAll = 32, kHead = 32 + (int)((sizeof(Groups) + 15) / 16 * 2);
+
+// ALL: the nets fit in LDS together (one group)
+template <class SH, bool ALL, int NW>
 __global__ void __launch_bounds__(64 * NW) k_fwd64(EmbArgs A) {
   extern __shared__ __align__(16) double sm[];
   double* tab = sm;                                     // [32]
-  double* scr = sm + 32;                                // [NW][kFwdScratch]
-  double* nets = scr + (size_t)NW * kFwdScratch<SH>;    // LDS: [nnets][SH::size]
+  Groups& groups = *reinterpret_cast<Groups*>(sm + kHeadAll);
+  double* scr = sm + (ALL ? kHeadAll : kHead);          // [NW][kFwdScratch]
+  double* nets = scr + (size_t)NW * kFwdScratch<SH>;    // [room][SH::size]
   if (threadIdx.x < 32) tab[threadIdx.x] = kExp2Tab[threadIdx.x];
-  if constexpr (LDS) stage_nets<SH>(nets, A.params, A.nnets);
-  __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int g = lane >> 4, c = lane & 15;
   const int per = NW / A.split, sub = wave % A.split, mine = wave / A.split;
@@ -312,96 +411,128 @@ __global__ void __launch_bounds__(64 * NW) k_fwd64(EmbArgs A) {
   const double* part = scr + (size_t)(wave - sub) * kFwdScratch<SH>;
   const double inv = 1.0 / (double)A.nnei;
   const int sn = 16 * SH::B3;  // channels of a partial row
-  for (int base = blockIdx.x * per; base < A.natoms; base += gridDim.x * per) {
-    const int atom = base + mine;
-    if (atom < A.natoms) {
-      const double* e = A.em + (size_t)atom * A.nnei * 4;
-      double acc[SH::B3], accy[SH::B2];
+  const bool dyn = !ALL && A.split == 1;
+  const int used = ALL ? A.nnets : list_nets(A, groups, per);
+  int p0 = 0, p1 = 0;
+  do {
+    p0 = p1;
+    p1 = ALL || p0 + A.room > used ? used : p0 + A.room;
+    if (!ALL) __syncthreads();  // the wavefronts are done with the nets before
+    stage_nets<SH, NW>(nets, A.params, ALL ? nullptr : groups.list, p0, p1, wave, lane);
+    __syncthreads();
+    // one turn: an atom for every `split` wavefronts, or (work false) none
+    auto turn = [&](int atom, bool work) {
+      int ti = 0;
+      unsigned blocks = ~0u;
+      bool earlier = false;
+      if (work) {
+        ti = A.atype[atom] < 0 ? 0 : A.atype[atom];
+        if constexpr (!ALL) blocks = group_blocks(A, groups, p0, p1, ti, earlier);
+      }
+      if (work) {
+        const double* e = A.em + (size_t)atom * A.nnei * 4;
+        double acc[SH::B3], accy[SH::B2];
 #pragma unroll
-      for (int m = 0; m < SH::B3; ++m) acc[m] = 0.0;
+        for (int m = 0; m < SH::B3; ++m) acc[m] = 0.0;
 #pragma unroll
-      for (int m = 0; m < SH::B2; ++m) accy[m] = 0.0;
-      for_tiles<false>(A, atom, sub, lane, [&](int k, int s0, int b1, int) {
-        asm volatile("" ::: "memory");  // weights are read every tile, not kept in registers
-        const Net<SH, LDS> net{LDS ? nets + (size_t)k * SH::size : A.params + (size_t)k * NET,
-                               lane};
-        const double s = s0 + c < b1 ? e[(s0 + c) * 4] : 0.0;
-        double rT[4];  // component c % 4 of slot 4 i + g
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int sl = s0 + 4 * i + g;
-          rT[i] = sl < b1 ? e[sl * 4 + (c & 3)] : 0.0;
-        }
-        double y2[SH::S2], none[1];
-        layers12<SH, LDS, false>(A, net, tab, s, g, y2, none);
-        if (!SH::G || A.res3 == 2) {
-#pragma unroll
-          for (int m = 0; m < SH::B2; ++m) {  // turn y2: slots on the registers
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              tile[c * 17 + 4 * i + g] = 4 * m + i < SH::S2 ? y2[4 * m + i < SH::S2 ? 4 * m + i : 0] : 0.0;
-            wave_sync();
-#pragma unroll
-            for (int i = 0; i < 4; ++i) accy[m] = mma4(rT[i], tile[(4 * i + g) * 17 + c], accy[m]);
-            wave_sync();
-          }
-        }
-#pragma unroll
-        for (int m = 0; m < SH::B3; ++m) {
-          const double b = net.b3(16 * m + c);
-          v4d z = {b, b, b, b};
-#pragma unroll
-          for (int ks = 0; ks < SH::S2; ++ks) z = mma16(y2[ks], net.w3(m, ks), z);
+        for (int m = 0; m < SH::B2; ++m) accy[m] = 0.0;
+        for_tiles<false>(A, atom, ti, blocks, sub, lane, [&](int k, int s0, int b1, int) {
+          asm volatile("" ::: "memory");  // weights are read every tile, not kept in registers
+          const Net<SH> net{nets + (size_t)((ALL ? k : groups.at[k]) - p0) * SH::size, lane};
+          const double s = s0 + c < b1 ? e[(s0 + c) * 4] : 0.0;
+          double rT[4];  // component c % 4 of slot 4 i + g
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            double f, d;
-            act64<SH, false>(A, tab, z[i], f, d);
-            if constexpr (SH::G) {
-              if (A.idt) f *= net.i3(16 * m + c);
-            }
-            acc[m] = mma4(rT[i], f, acc[m]);
+            const int sl = s0 + 4 * i + g;
+            rT[i] = sl < b1 ? e[sl * 4 + (c & 3)] : 0.0;
           }
-          net.fence();
-        }
-      });
-      if (A.pad != nullptr && A.nlist != nullptr && sub == 0 && A.atype[atom] >= 0) {
-        const int ti = A.atype[atom];
-        for (int t = 0; t < A.ntypes; ++t) {
-          const int b1 = block_end(A.nlist + (size_t)atom * A.nnei, A.sec[t], A.sec[t + 1], lane);
-          if (b1 >= A.sec[t + 1]) continue;
-          const double* pt = A.pad + (((size_t)ti * A.nnei + b1) * 4 + g) * P3;
+          double y2[SH::S2], none[1];
+          layers12<SH, false>(A, net, tab, s, g, y2, none);
+          if (!SH::G || A.res3 == 2) {
 #pragma unroll
-          for (int m = 0; m < SH::B3; ++m) acc[m] += pt[SH::inner(16 * m + c)];
+            for (int m = 0; m < SH::B2; ++m) {  // turn y2: slots on the registers
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                tile[c * 17 + 4 * i + g] = 4 * m + i < SH::S2 ? y2[4 * m + i < SH::S2 ? 4 * m + i : 0] : 0.0;
+              wave_sync();
+#pragma unroll
+              for (int i = 0; i < 4; ++i) accy[m] = mma4(rT[i], tile[(4 * i + g) * 17 + c], accy[m]);
+              wave_sync();
+            }
+          }
+#pragma unroll
+          for (int m = 0; m < SH::B3; ++m) {
+            const double b = net.b3(16 * m + c);
+            v4d z = {b, b, b, b};
+#pragma unroll
+            for (int ks = 0; ks < SH::S2; ++ks) z = mma16(y2[ks], net.w3(m, ks), z);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              double f, d;
+              act64<SH, false>(A, tab, z[i], f, d);
+              if constexpr (SH::G) {
+                if (A.idt) f *= net.i3(16 * m + c);
+              }
+              acc[m] = mma4(rT[i], f, acc[m]);
+            }
+            net.fence();
+          }
+        });
+        if (A.pad != nullptr && A.nlist != nullptr && sub == 0 && A.atype[atom] >= 0) {
+          for (int t = 0; t < A.ntypes; ++t) {
+            if (!(blocks >> t & 1)) continue;
+            const int b1 = block_end(A.nlist + (size_t)atom * A.nnei, A.sec[t], A.sec[t + 1], lane);
+            if (b1 >= A.sec[t + 1]) continue;
+            const double* pt = A.pad + (((size_t)ti * A.nnei + b1) * 4 + g) * P3;
+#pragma unroll
+            for (int m = 0; m < SH::B3; ++m) acc[m] += pt[SH::inner(16 * m + c)];
+          }
+        }
+        // lane (g, c): component g, channels 16 m + c of the wavefront's tiles;
+        // the resnet part of channel n is that of channel n mod 4 S2 of y2
+#pragma unroll
+        for (int m = 0; m < SH::B3; ++m) tile[g * sn + 16 * m + c] = acc[m];
+        wave_sync();
+#pragma unroll
+        for (int m = 0; m < SH::B2; ++m) {
+          const int n = 16 * m + c;
+          if (n < 4 * SH::S2) {
+            tile[g * sn + n] += accy[m];
+            tile[g * sn + n + 4 * SH::S2] += accy[m];
+          }
         }
       }
-      // lane (g, c): component g, channels 16 m + c of the wavefront's tiles;
-      // the resnet part of channel n is that of channel n mod 4 S2 of y2
-#pragma unroll
-      for (int m = 0; m < SH::B3; ++m) tile[g * sn + 16 * m + c] = acc[m];
-      wave_sync();
-#pragma unroll
-      for (int m = 0; m < SH::B2; ++m) {
-        const int n = 16 * m + c;
-        if (n < 4 * SH::S2) {
-          tile[g * sn + n] += accy[m];
-          tile[g * sn + n + 4 * SH::S2] += accy[m];
+      if (A.split > 1) __syncthreads();
+      else wave_sync();
+      if (work) {
+        double* o = A.out + (size_t)atom * 4 * A.d3;
+        for (int q = sub * 64 + lane; q < 4 * sn; q += 64 * A.split) {
+          double v = 0.0;
+          for (int w = 0; w < A.split; ++w) v += part[(size_t)w * kFwdScratch<SH> + q];
+          const int tc = A.ch_out[SH::inner(q % sn)];
+          if (tc < 0) continue;
+          double* r = o + (q / sn) * A.d3 + tc;
+          *r = earlier ? *r + v * inv : v * inv;
         }
+      }
+      if (A.split > 1) __syncthreads();
+      else wave_sync();
+    };
+    if constexpr (ALL) {
+      for (int base = blockIdx.x * per; base < A.natoms; base += gridDim.x * per)
+        turn(base + mine, base + mine < A.natoms);
+    } else {
+      const unsigned types = group_types(A, groups, p0, p1, lane);
+      int dealt = 0;  // whole atoms go to the wavefronts in turn
+      for (int q0 = 0; atom_at(q0, per) < A.natoms; q0 += 64) {
+        const unsigned long long m = atoms_of(A, types, q0, per, lane);
+        const int n = __popcll(m), off = A.split == 1 ? (mine - dealt) & (per - 1) : mine;
+        for (int i = 0; i < n; i += per)
+          turn(atom_at(q0 + nth_bit(m, i + off < n ? i + off : 0), per), i + off < n);
+        dealt += n;
       }
     }
-    if (A.split > 1) __syncthreads();
-    else wave_sync();
-    if (atom < A.natoms) {
-      double* o = A.out + (size_t)atom * 4 * A.d3;
-      for (int q = sub * 64 + lane; q < 4 * sn; q += 64 * A.split) {
-        double v = 0.0;
-        for (int w = 0; w < A.split; ++w) v += part[(size_t)w * kFwdScratch<SH> + q];
-        const int tc = A.ch_out[SH::inner(q % sn)];
-        if (tc >= 0) o[(q / sn) * A.d3 + tc] = v * inv;
-      }
-    }
-    if (A.split > 1) __syncthreads();
-    else wave_sync();
-  }
+  } while (!ALL && p1 < used);
 }
 
 // -------------------------------------------------------------- backward --
@@ -410,90 +541,122 @@ __global__ void __launch_bounds__(64 * NW) k_fwd64(EmbArgs A) {
 template <class SH>
 constexpr int kGs = 16 * SH::B3 + 4;
 
-template <class SH, bool LDS, int NW>
+template <class SH, bool ALL, int NW>
 __global__ void __launch_bounds__(64 * NW) k_bwd64(EmbArgs A) {
   extern __shared__ __align__(16) double sm[];
   double* tab = sm;
-  double* scr = sm + 32;
+  Groups& groups = *reinterpret_cast<Groups*>(sm + kHeadAll);
+  double* scr = sm + (ALL ? kHeadAll : kHead);
   double* nets = scr + (size_t)NW * 4 * kGs<SH>;
   if (threadIdx.x < 32) tab[threadIdx.x] = kExp2Tab[threadIdx.x];
-  if constexpr (LDS) stage_nets<SH>(nets, A.params, A.nnets);
-  __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int g = lane >> 4, c = lane & 15;
   double* gx = scr + (size_t)wave * 4 * kGs<SH>;
   const double inv = 1.0 / (double)A.nnei;
   const long units = (long)A.natoms * A.split;
-  for (long u = (long)blockIdx.x * NW + wave; u < units; u += (long)gridDim.x * NW) {
-    // (the turn of the parts goes round: a wavefront's units are all sizes)
-    const int atom = (int)(u / A.split), sub = (int)((u + atom) % A.split);
-    const double* e = A.em + (size_t)atom * A.nnei * 4;
-    double* nd = A.out + (size_t)atom * A.nnei * 4;
-    wave_sync();
-    for (int q = lane; q < 4 * 16 * SH::B3; q += 64) {
-      const int n = q % (16 * SH::B3), cc = q / (16 * SH::B3), tc = A.ch_out[SH::inner(n)];
-      gx[cc * kGs<SH> + n] =
-          tc >= 0 ? A.gxyz[(size_t)atom * 4 * A.d3 + cc * A.d3 + tc] * inv : 0.0;
-    }
-    wave_sync();
-    for_tiles<true>(A, atom, sub, lane, [&](int k, int s0, int b1, int end) {
-      asm volatile("" ::: "memory");  // weights are read every tile, not kept in registers
-      const Net<SH, LDS> net{LDS ? nets + (size_t)k * SH::size : A.params + (size_t)k * NET,
-                             lane};
-      const int slot = s0 + c;
-      const double s = slot < b1 ? e[slot * 4] : 0.0;
-      double y2[SH::S2], d2[SH::S2];
-      layers12<SH, LDS, true>(A, net, tab, s, g, y2, d2);
-      double dR = 0.0, Mx = 0.0;  // component g of slot c
+  const int used = ALL ? A.nnets : list_nets(A, groups, NW / A.split);
+  int p0 = 0, p1 = 0;
+  do {
+    p0 = p1;
+    p1 = ALL || p0 + A.room > used ? used : p0 + A.room;
+    if (!ALL) __syncthreads();
+    stage_nets<SH, NW>(nets, A.params, ALL ? nullptr : groups.list, p0, p1, wave, lane);
+    __syncthreads();
+    // part `sub` of an atom's tiles
+    auto unit = [&](int atom, int sub) {
+      const int ti = A.atype[atom] < 0 ? 0 : A.atype[atom];
+      unsigned blocks = ~0u;
+      if constexpr (!ALL) {
+        bool earlier;
+        blocks = group_blocks(A, groups, p0, p1, ti, earlier);
+      }
+      const double* e = A.em + (size_t)atom * A.nnei * 4;
+      double* nd = A.out + (size_t)atom * A.nnei * 4;
+      wave_sync();
+      for (int q = lane; q < 4 * 16 * SH::B3; q += 64) {
+        const int n = q % (16 * SH::B3), cc = q / (16 * SH::B3), tc = A.ch_out[SH::inner(n)];
+        gx[cc * kGs<SH> + n] =
+            tc >= 0 ? A.gxyz[(size_t)atom * 4 * A.d3 + cc * A.d3 + tc] * inv : 0.0;
+      }
+      wave_sync();
+      for_tiles<true>(A, atom, ti, blocks, sub, lane, [&](int k, int s0, int b1, int end) {
+        asm volatile("" ::: "memory");  // weights are read every tile, not kept in registers
+        const Net<SH> net{nets + (size_t)((ALL ? k : groups.at[k]) - p0) * SH::size, lane};
+        const int slot = s0 + c;
+        const double s = slot < b1 ? e[slot * 4] : 0.0;
+        double y2[SH::S2], d2[SH::S2];
+        layers12<SH, true>(A, net, tab, s, g, y2, d2);
+        double dR = 0.0, Mx = 0.0;  // component g of slot c
 #pragma unroll
-      for (int m = 0; m < SH::B3; ++m) {
-        v4d z, dz = {0.0, 0.0, 0.0, 0.0};
+        for (int m = 0; m < SH::B3; ++m) {
+          v4d z, dz = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) z[i] = net.b3(16 * m + 4 * i + g);
+          for (int i = 0; i < 4; ++i) z[i] = net.b3(16 * m + 4 * i + g);
 #pragma unroll
-        for (int ks = 0; ks < SH::S2; ++ks) {
-          const double w = net.w3(m, ks);
-          z = mma16(w, y2[ks], z);
-          dz = mma16(w, d2[ks], dz);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int t = (4 * m + i) % SH::S2;
-          double f, d;
-          act64<SH, true>(A, tab, z[i], f, d);
-          if constexpr (SH::G) {
-            d *= dz[i];
-            if (A.idt) {
-              const double ts = net.i3(16 * m + 4 * i + g);
-              f *= ts;
-              d *= ts;
-            }
-            if (A.res3 == 2) {
-              f += y2[t];
-              d += d2[t];
-            }
-          } else {
-            f += y2[t];
-            d = __fma_rn(d, dz[i], d2[t]);
+          for (int ks = 0; ks < SH::S2; ++ks) {
+            const double w = net.w3(m, ks);
+            z = mma16(w, y2[ks], z);
+            dz = mma16(w, d2[ks], dz);
           }
-          const double ga = gx[(c & 3) * kGs<SH> + 16 * m + 4 * i + g];
-          dR = mma4(ga, f, dR);
-          Mx = mma4(ga, d, Mx);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int t = (4 * m + i) % SH::S2;
+            double f, d;
+            act64<SH, true>(A, tab, z[i], f, d);
+            if constexpr (SH::G) {
+              d *= dz[i];
+              if (A.idt) {
+                const double ts = net.i3(16 * m + 4 * i + g);
+                f *= ts;
+                d *= ts;
+              }
+              if (A.res3 == 2) {
+                f += y2[t];
+                d += d2[t];
+              }
+            } else {
+              f += y2[t];
+              d = __fma_rn(d, dz[i], d2[t]);
+            }
+            const double ga = gx[(c & 3) * kGs<SH> + 16 * m + 4 * i + g];
+            dR = mma4(ga, f, dR);
+            Mx = mma4(ga, d, Mx);
+          }
+          net.fence();
         }
-        net.fence();
+        const double R = slot < b1 ? e[slot * 4 + g] : 0.0;
+        double ds = R * Mx;
+        ds += __shfl_xor(ds, 16, 64);
+        ds += __shfl_xor(ds, 32, 64);
+        const double v = g == 0 ? dR + ds : dR;
+        if (slot < b1) nd[slot * 4 + g] = v;
+        if (end > b1 && b1 <= s0 + 16) {  // slot b1 - 1 stands for the padding after it
+          const double w = __shfl(v, 16 * g + (b1 - 1 - s0), 64);
+          for (int q = b1 + c; q < end; q += 16) nd[q * 4 + g] = w;
+        }
+      });
+    };
+    // (the turn of the parts goes round: a wavefront's units are all sizes)
+    if constexpr (ALL) {
+      for (long u = (long)blockIdx.x * NW + wave; u < units; u += (long)gridDim.x * NW) {
+        const int atom = (int)(u / A.split);
+        unit(atom, (int)((u + atom) % A.split));
       }
-      const double R = slot < b1 ? e[slot * 4 + g] : 0.0;
-      double ds = R * Mx;
-      ds += __shfl_xor(ds, 16, 64);
-      ds += __shfl_xor(ds, 32, 64);
-      const double v = g == 0 ? dR + ds : dR;
-      if (slot < b1) nd[slot * 4 + g] = v;
-      if (end > b1 && b1 <= s0 + 16) {  // slot b1 - 1 stands for the padding after it
-        const double w = __shfl(v, 16 * g + (b1 - 1 - s0), 64);
-        for (int q = b1 + c; q < end; q += 16) nd[q * 4 + g] = w;
+    } else {
+      const unsigned types = group_types(A, groups, p0, p1, lane);
+      const int per = NW / A.split;
+      int dealt = 0;
+      for (int q0 = 0; atom_at(q0, per) < A.natoms; q0 += 64) {
+        const unsigned long long m = atoms_of(A, types, q0, per, lane);
+        const int n = __popcll(m) * A.split;
+        for (int i = (wave - dealt) & (NW - 1); i < n; i += NW) {
+          const int atom = atom_at(q0 + nth_bit(m, i / A.split), per);
+          unit(atom, (i + atom) % A.split);
+        }
+        dealt += n;
       }
-    });
-  }
+    }
+  } while (!ALL && p1 < used);
 }
 
 constexpr int kLdsMax = 160 * 1024;
@@ -509,12 +672,21 @@ constexpr int kWaves = 8;
 // wavefronts, and with many a finer split evens out the last round (5,324 Cu
 // atoms of 12 tiles on 2,048 wavefronts: 3 rounds of 12 tiles whole, 11 of 3
 // split by four).  Tiles an atom: sel is set about a tenth above the
-// neighbours a system has.
-int choose_split(int natoms, int tiles, int waves) {
+// neighbours a system has.  Nets in groups: a group's blocks may hold any
+// number of tiles, so the atoms that use a group (all, or with a net a centre
+// and neighbour type `share` of them) are split only while the chip is not full.
+int choose_split(const EmbArgs& A, int tiles, int ncu) {
+  const long waves = (long)ncu * kWaves;
   int best = 1;
+  if (A.room < A.nnets) {
+    const bool pairs = A.nnets > A.ntypes;  // a net a centre and neighbour type
+    const double share = pairs && A.room < A.ntypes ? (double)A.room / A.ntypes : 1.0;
+    while (best < kWaves && A.natoms * share * 2 * best <= (double)waves) best *= 2;
+    return best;
+  }
   long cost = -1;
   for (int s = 1; s <= kWaves; s *= 2) {
-    const long c = (((long)natoms * s + waves - 1) / waves) * ((tiles + s - 1) / s);
+    const long c = (((long)A.natoms * s + waves - 1) / waves) * ((tiles + s - 1) / s);
     if (cost < 0 || c < cost) {
       cost = c;
       best = s;
@@ -523,7 +695,7 @@ int choose_split(int natoms, int tiles, int waves) {
   return best;
 }
 
-template <class SH, bool LDS>
+template <class SH>
 int launch64(bool fwd, EmbArgs& A, hipStream_t st) {
   constexpr int NW = kWaves;
   static int ncu[64];
@@ -532,31 +704,24 @@ int launch64(bool fwd, EmbArgs& A, hipStream_t st) {
   DPK_REQUIRE(dev >= 0 && dev < 64, DPK_ERR_ARG, "embed: device %d out of range", dev);
   if (ncu[dev] == 0)
     DPK_HIP(hipDeviceGetAttribute(&ncu[dev], hipDeviceAttributeMultiprocessorCount, dev));
+  constexpr int kMost = NW * (kFwdScratch<SH> > 4 * kGs<SH> ? kFwdScratch<SH> : 4 * kGs<SH>);
+  constexpr int kRoom = (kLdsMax / 8 - kHead - kMost) / SH::size;
+  static_assert(kRoom >= 1, "a net fits in LDS beside the scratch");
+  A.room = kRoom < A.nnets ? kRoom : A.nnets;
+  const bool all = A.room == A.nnets;
   const size_t lds =
-      sizeof(double) * (32 + (size_t)NW * (fwd ? kFwdScratch<SH> : 4 * kGs<SH>) +
-                        (LDS ? (size_t)A.nnets * SH::size : 0));
+      sizeof(double) * ((all ? kHeadAll : kHead) + (size_t)NW * (fwd ? kFwdScratch<SH> : 4 * kGs<SH>) +
+                        (size_t)A.room * SH::size);
   int tiles = 0;
   for (int t = 0; t < A.ntypes; ++t) tiles += (9 * (A.sec[t + 1] - A.sec[t]) / 10 + 15) / 16;
-  A.split = choose_split(A.natoms, tiles, ncu[dev] * NW);
+  A.split = choose_split(A, tiles, ncu[dev]);
   const long want = ((long)A.natoms * A.split + NW - 1) / NW;
-  // LDS: one workgroup a CU; without, the register budget's two
-  const long room = (long)ncu[dev] * (LDS ? 1 : 2);
-  const unsigned grid = (unsigned)(want < room ? want : room);
-  if (fwd)
-    hipLaunchKernelGGL((k_fwd64<SH, LDS, NW>), dim3(grid), dim3(64 * NW), lds, st, A);
-  else
-    hipLaunchKernelGGL((k_bwd64<SH, LDS, NW>), dim3(grid), dim3(64 * NW), lds, st, A);
+  const unsigned grid = (unsigned)(want < ncu[dev] ? want : ncu[dev]);  // one workgroup a CU
+  const auto kernel = fwd ? (all ? k_fwd64<SH, true, NW> : k_fwd64<SH, false, NW>)
+                          : (all ? k_bwd64<SH, true, NW> : k_bwd64<SH, false, NW>);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * NW), lds, st, A);
   DPK_LAUNCHED();
   return DPK_OK;
-}
-
-template <class SH>
-int launch_shape(bool fwd, EmbArgs& A, hipStream_t st) {
-  const size_t most = 32 + (size_t)kWaves * (kFwdScratch<SH> > 4 * kGs<SH> ? kFwdScratch<SH>
-                                                                            : 4 * kGs<SH>);
-  if (sizeof(double) * (most + (size_t)A.nnets * SH::size) <= kLdsMax)
-    return launch64<SH, true>(fwd, A, st);
-  return launch64<SH, false>(fwd, A, st);
 }
 
 }  // namespace
@@ -586,12 +751,13 @@ int embed_f64(bool fwd, void* out, const void* em, const void* gx, const int* at
   A.idt = has_idt;
   A.act = act;
   for (int t = 0; t <= ntypes; ++t) A.sec[t] = sec_host[t];
-  if (act.id != DPK_ACT_TANH || has_idt || res2 != 2 || res3 != 2)
-    return launch_shape<Shape<8, true>>(fwd, A, st);
+  A.room = nnets;
+  if (act.id != DPK_ACT_TANH) return launch64<Shape<8, kAny>>(fwd, A, st);
+  if (has_idt || res2 != 2 || res3 != 2) return launch64<Shape<8, kTanh>>(fwd, A, st);
   // doubling resnets: d3 = 4 d1, so d3 <= 112 leaves the eighth step of every
   // copy empty
-  if (d3 <= 112) return launch_shape<Shape<7, false>>(fwd, A, st);
-  return launch_shape<Shape<8, false>>(fwd, A, st);
+  if (d3 <= 112) return launch64<Shape<7, kPlain>>(fwd, A, st);
+  return launch64<Shape<8, kPlain>>(fwd, A, st);
 }
 
 }  // namespace dpk

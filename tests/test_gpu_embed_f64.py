@@ -1,5 +1,5 @@
 """FP64 embedding kernels (csrc/embed_f64.hip) on their own, against the oracle's
-descriptor contraction and its autograd: nets in LDS and read from memory,
+descriptor contraction and its autograd: nets in LDS together and in groups,
 seven and eight channel steps, one wavefront an atom and several (few atoms),
 block lengths around the 16-slot tile, and the padding left out or not."""
 
@@ -82,12 +82,12 @@ def _check(got, ref, what):
 @pytest.mark.parametrize("neuron,sel,one_side,natoms,extra", [
     ([25, 50, 100], [46, 92], True, 7, {}),           # two nets in LDS, eight wavefronts an atom
     ([25, 50, 100], [46, 92], True, 1100, {}),        # two nets in LDS, one wavefront an atom
-    ([25, 50, 100], [17, 15], False, 40, {}),         # four nets, from memory
+    ([25, 50, 100], [17, 15], False, 40, {}),         # four nets, two at a time
     ([28, 56, 112], [16], True, 1, {}),               # the widest of seven steps
     ([29, 58, 116], [33], True, 130, {}),             # the narrowest of eight
     ([32, 64, 128], [200], True, 600, {}),
     ([10, 20, 40], [1, 31], True, 9, {}),
-    ([32, 64, 128], [20, 20], True, 30, {}),          # two wide nets: from memory
+    ([32, 64, 128], [20, 20], True, 30, {}),          # two wide nets, one at a time
     ([25, 50, 100], [30], True, 50, {"act": "gelu"}),
     ([25, 50, 100], [30, 20], True, 50, {"act": "silut:2.5", "dt": True}),
     ([20, 30, 100], [40], True, 50, {}),              # no doubling: no resnet copies
@@ -132,3 +132,28 @@ def test_embed_f64_nan_and_infinity():
     ref, _ = _oracle(d, at, em, gx)
     assert np.array_equal(np.isfinite(x[4]), np.isfinite(ref[4]))
     _check(x[4, 1:], ref[4, 1:], "components with a finite row")
+
+
+@pytest.mark.parametrize("neuron,sel,one_side,natoms,extra", [
+    ([32, 64, 128], [20, 9, 14], False, 61, {}),      # nine nets: a workgroup lists those it uses
+    ([25, 50, 100], [17, 15], False, 2100, {}),       # more atoms than wavefronts
+    ([32, 64, 128], [33, 18], True, 1100, {}),        # all atoms in both groups, whole and split
+    ([32, 64, 128], [33, 18], True, 300, {}),
+    ([32, 64, 128], [2, 3], False, 16500, {}),        # more than 64 atoms a workgroup
+    ([20, 30, 100], [30, 20], False, 700, {"dt": True}),
+    ([25, 50, 100], [30, 20], False, 600, {"act": "gelu"}),
+])
+def test_embed_f64_nets_in_groups(neuron, sel, one_side, natoms, extra):
+    """Nets that don't fit in LDS together; every seventh atom is virtual (its
+    rows are zero and its list is empty: zero in the forward, the derivative of
+    type 0 in the backward)."""
+    d, at, em, nl, gx = _case(neuron, sel, one_side, natoms, **extra)
+    em[3::7], nl[3::7] = 0.0, -1
+    real = at.copy()
+    at[3::7], real[3::7] = -1, 0
+    xyz, nd = _oracle(d, real, em, gx)
+    for skip in (True, False):
+        x, n = _run(d, at, em, nl, gx, skip)
+        _check(x, xyz, f"xyz {neuron} {sel} n={natoms} skip={skip}")
+        _check(n, nd, f"net_deriv {neuron} {sel} n={natoms} skip={skip}")
+        assert not x[3::7].any()
