@@ -84,7 +84,7 @@ struct dpk_deeppot {
   int nloc = -1, nall = -1, nnei_in = -1, nreal = 0;
   std::vector<int> seg_type, seg_start, seg_end;
   DevBuf coord, atype, nlist_in, nlist, status, em, xyz, gxyz, atom_e, nd, force, vrow, virial,
-      energy, fsum_ws, frame_of, frames, sums, shift, order, z1, gz, gather_ws;
+      energy, fsum_ws, frame_of, frames, sums, shift, order, z1, gz;
   bool have_list = false;
 };
 
@@ -269,7 +269,6 @@ bool setup(dpk_deeppot* dp, const int* atype, int nall, int nloc, int inum, cons
             dp->gxyz.reserve(sizeof(float) * nl1 * 4 * d3) && dp->atom_e.reserve(sizeof(double) * nl1) &&
             dp->nd.reserve(sizeof(float) * nl1 * S * 4) && dp->force.reserve(sizeof(double) * 3 * nall) &&
             dp->vrow.reserve(dpk_force_virial_workspace_bytes(nloc)) &&
-            dp->gather_ws.reserve(dpk_force_virial_gather_workspace_bytes(nloc, S, nall)) &&
             dp->virial.reserve(sizeof(double) * 9) && dp->energy.reserve(sizeof(double)) &&
             dp->fsum_ws.reserve(dpk_frame_sum_workspace_bytes(1, nloc, 9)) &&
             dp->frame_of.reserve(sizeof(int) * nl1) && dp->frames.reserve(sizeof(dpk_frame)) &&
@@ -368,14 +367,14 @@ bool step(dpk_deeppot* dp, const double* coord, bool check_list, double* energy,
       !hip_ok(hipMemsetAsync(dp->force.p, 0, sizeof(double) * 3 * nall, st), "memset"))
     return false;
   if (nloc) {
-    // neighbour forces gathered per extended atom (writes every force row)
+    // (writes every force row; a workspace is for the atomic virial only)
     if (!dpk_ok(dpk_force_virial_gather(dp->force.as<double>(), nullptr,
                                         static_cast<double*>(dp->vrow.p), dp->nd.p, dp->prec,
                                         dp->coord.as<double>(), dp->atype.as<int>(),
                                         dp->nlist.as<int>(),
                                         static_cast<const double*>(bp(dp, "dstd")), nloc, S, nall,
                                         dp->rcut, dp->rcut_smth, dp->protection, pm, dp->ntypes,
-                                        dp->gather_ws.p, dp->gather_ws.n, s),
+                                        nullptr, 0, s),
                 "dpk_force_virial_gather") ||
         !dpk_ok(dpk_frame_sum(dp->virial.as<double>(), static_cast<const double*>(dp->vrow.p), 9,
                               dp->sums.as<dpk_frame>(), 1, nloc, dp->fsum_ws.p, dp->fsum_ws.n, s),

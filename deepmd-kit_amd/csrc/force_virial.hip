@@ -475,10 +475,13 @@ int frame_sum_t(double* out, const double* in, const dpk_frame* frames, int nfra
 
 // --------------------------------------------------------------- MD path --
 // For an engine's extended region (explicit ghosts: the list holds
-// extended-atom indices).  One wavefront per centre: its neighbours' shares
-// are added to force (and, on request, the atomic virial) by rows
-// (add_rows), the centre's -sum and its virial row vrow[centre] = sum f (x) d
-// are summed in registers.  force and atom_virial are cleared before.
+// extended-atom indices), in one of two forms (gather_pays):
+//
+// Added.  One wavefront per centre: its neighbours' shares are added to force
+// (and, on request, the atomic virial) by rows (add_rows), the centre's -sum
+// and its virial row vrow[centre] = sum f (x) d are summed in registers.  force
+// and atom_virial are cleared before.  Bound by the FP64 atomics, three or
+// twelve a slot.
 template <typename GT>
 __global__ void __launch_bounds__(256) k_slot_add(
     double* __restrict__ force, double* __restrict__ atom_virial, double* __restrict__ vrow,
@@ -541,6 +544,159 @@ __global__ void __launch_bounds__(256) k_slot_add(
   for (int k = 0; k < 9; ++k) {
     const double t = wave_sum(vacc[k]);
     if (lane == 0) vrow[(size_t)g * 9 + k] = t;
+  }
+}
+
+// Gathered.  The slots are binned by neighbour into fixed-capacity buckets (cap
+// ~ the slot count: an atom is a neighbour of about as many centres as it has
+// neighbours; slots beyond a full bucket go to an overflow list, added with
+// atomics at the end), one pass writes every slot's force share f (summing the
+// centre's -f and virial row in registers), a second pass sums each extended
+// atom's bucket.  Bound by the passes over the shares, 28 bytes a slot, and
+// hardly dearer with the atomic virial.
+
+__global__ void k_bucket_zero(int* __restrict__ count, int n) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q <= n) count[q] = 0;  // count[n]: the overflow length
+}
+
+// the slot's neighbour (or -1: empty, outside the region, excluded pair)
+__device__ __forceinline__ int gather_nbr(const int* __restrict__ nlist,
+                                          const int* __restrict__ atype,
+                                          const int* __restrict__ pair_mask, int ntypes,
+                                          long long s, int nnei, int nall) {
+  const int e = nlist[s];
+  if (e < 0 || e >= nall) return -1;
+  if (pair_mask != nullptr) {
+    const int traw = atype[(int)(s / nnei)];
+    const int* pm = pair_mask + (traw < 0 ? ntypes : traw) * (ntypes + 1);
+    const int tj = atype[e];
+    if (!pm[tj < 0 ? ntypes : tj]) return -1;
+  }
+  return e;
+}
+
+__global__ void k_bucket_fill(int* __restrict__ bucket, int* __restrict__ count,
+                              int* __restrict__ ovf, const int* __restrict__ nlist,
+                              const int* __restrict__ atype, const int* __restrict__ pair_mask,
+                              int ntypes, long long total, int nnei, int nall, int cap) {
+  const long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= total) return;
+  const int e = gather_nbr(nlist, atype, pair_mask, ntypes, s, nnei, nall);
+  if (e < 0) return;
+  const int pos = atomicAdd(count + e, 1);
+  if (pos < cap) bucket[(size_t)e * cap + pos] = (int)s;
+  else ovf[atomicAdd(count + nall, 1)] = (int)s;
+}
+
+// One wavefront per centre: fs[slot] = the force share of the slot's
+// neighbour, force[centre] = -sum of them, vrow[centre] = sum f (x) d.
+template <typename GT>
+__global__ void __launch_bounds__(256) k_slot_forces(
+    double* __restrict__ fs, double* __restrict__ force, double* __restrict__ vrow,
+    const GT* __restrict__ nd, const double* __restrict__ coord, const int* __restrict__ atype,
+    const int* __restrict__ nlist, const double* __restrict__ stdv, int natoms, int nnei,
+    int nall, double rcut, double rcut_smth, double protection,
+    const int* __restrict__ pair_mask, int ntypes) {
+  const int g = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (g >= natoms) return;
+  const int traw = atype[g];
+  const int ti = traw < 0 ? 0 : traw;
+  const double cx = coord[3 * g], cy = coord[3 * g + 1], cz = coord[3 * g + 2];
+  double ci[3] = {0.0, 0.0, 0.0};
+  double vacc[9];
+  for (int k = 0; k < 9; ++k) vacc[k] = 0.0;
+  for (int jj = lane; jj < nnei; jj += kWave) {
+    const size_t s = (size_t)g * nnei + jj;
+    const int j = gather_nbr(nlist, atype, pair_mask, ntypes, (long long)s, nnei, nall);
+    double f[3] = {0.0, 0.0, 0.0};
+    if (j >= 0) {
+      const double dd[3] = {coord[3 * j] - cx, coord[3 * j + 1] - cy, coord[3 * j + 2] - cz};
+      const double r = norm3_ref(dd[0], dd[1], dd[2]);
+      double sw, dsw;
+      spline5<double>(r, rcut_smth, rcut, sw, dsw);
+      const double inr = 1.0 / r;
+      const double iu = protection == 0.0 ? inr : 1.0 / (r + protection);
+      const double* sd = stdv + (size_t)ti * nnei * 4 + jj * 4;
+      double gg[4];
+      for (int c = 0; c < 4; ++c) gg[c] = (double)nd[s * 4 + c] / sd[c];
+      env_centre_deriv<double>(dd, inr, iu, sw, dsw, gg, f);
+      for (int a = 0; a < 3; ++a) {
+        ci[a] -= f[a];
+        for (int b = 0; b < 3; ++b) vacc[3 * a + b] += f[a] * dd[b];
+      }
+    }
+    for (int a = 0; a < 3; ++a) fs[3 * s + a] = f[a];
+  }
+  for (int a = 0; a < 3; ++a) {
+    double t = wave_sum(ci[a]);
+    if (lane == 0) force[3 * (size_t)g + a] = t;
+  }
+  for (int k = 0; k < 9; ++k) {
+    double t = wave_sum(vacc[k]);
+    if (lane == 0) vrow[(size_t)g * 9 + k] = t;
+  }
+}
+
+// One wavefront per extended atom j: force[j] (= its centre part when j is
+// local, else 0) + the sum of its bucket's shares; atom_virial[j]
+// (optional) = sum f (x) (x_j - x_centre) over them.
+__global__ void __launch_bounds__(256) k_gather_forces(
+    double* __restrict__ force, double* __restrict__ atom_virial, const double* __restrict__ fs,
+    const int* __restrict__ count, const int* __restrict__ bucket,
+    const double* __restrict__ coord, int natoms, int nnei, int nall, int cap) {
+  const int j = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (j >= nall) return;
+  const int n = count[j] < cap ? count[j] : cap;
+  const int* row = bucket + (size_t)j * cap;
+  double f[3] = {0.0, 0.0, 0.0}, v[9];
+  for (int k = 0; k < 9; ++k) v[k] = 0.0;
+  const double xj = coord[3 * j], yj = coord[3 * j + 1], zj = coord[3 * j + 2];
+  for (int q = lane; q < n; q += kWave) {
+    const int s = row[q];
+    const double fx = fs[3 * (size_t)s], fy = fs[3 * (size_t)s + 1], fz = fs[3 * (size_t)s + 2];
+    f[0] += fx;
+    f[1] += fy;
+    f[2] += fz;
+    if (atom_virial != nullptr) {
+      const int i = s / nnei;
+      const double d[3] = {xj - coord[3 * i], yj - coord[3 * i + 1], zj - coord[3 * i + 2]};
+      const double ff[3] = {fx, fy, fz};
+      for (int a = 0; a < 3; ++a)
+        for (int b = 0; b < 3; ++b) v[3 * a + b] += ff[a] * d[b];
+    }
+  }
+  for (int a = 0; a < 3; ++a) {
+    const double t = wave_sum(f[a]);
+    if (lane == 0) force[3 * (size_t)j + a] = (j < natoms ? force[3 * (size_t)j + a] : 0.0) + t;
+  }
+  if (atom_virial != nullptr)
+    for (int k = 0; k < 9; ++k) {
+      const double t = wave_sum(v[k]);
+      if (lane == 0) atom_virial[9 * (size_t)j + k] = t;
+    }
+}
+
+// Slots that did not fit their bucket (count[nall] of them): added with
+// atomics, grid-stride over the device-side count.
+__global__ void k_gather_overflow(double* __restrict__ force, double* __restrict__ atom_virial,
+                                  const double* __restrict__ fs, const int* __restrict__ count,
+                                  const int* __restrict__ ovf, const int* __restrict__ nlist,
+                                  const double* __restrict__ coord, int nnei, int nall) {
+  const int n = count[nall];
+  for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += gridDim.x * blockDim.x) {
+    const int s = ovf[q];
+    const int j = nlist[s], i = s / nnei;
+    const double ff[3] = {fs[3 * (size_t)s], fs[3 * (size_t)s + 1], fs[3 * (size_t)s + 2]};
+    for (int a = 0; a < 3; ++a) atomicAdd(force + 3 * (size_t)j + a, ff[a]);
+    if (atom_virial != nullptr) {
+      const double d[3] = {coord[3 * j] - coord[3 * i], coord[3 * j + 1] - coord[3 * i + 1],
+                           coord[3 * j + 2] - coord[3 * i + 2]};
+      for (int a = 0; a < 3; ++a)
+        for (int b = 0; b < 3; ++b) atomicAdd(atom_virial + 9 * (size_t)j + 3 * a + b, ff[a] * d[b]);
+    }
   }
 }
 
@@ -622,9 +778,39 @@ extern "C" int dpk_prod_virial_grad_a_f64(double* grad_net, const double* grad,
   return DPK_OK;
 }
 
+// Workspace of the gathered form: count (nall + 1 ints, the last the
+// overflow length), buckets (nall * cap ints), the overflow list and the
+// force shares (natoms * nnei ints / doubles x 3); cap = nnei rounded up to 64.
+static int gather_cap(int nnei) { return (nnei + 63) / 64 * 64; }
+static size_t gather_ws_bytes(int natoms, int nnei, int nall, size_t* off_b, size_t* off_o,
+                              size_t* off_fs) {
+  const size_t slots = (size_t)natoms * (size_t)nnei;
+  auto al = [](size_t o) { return (o + 255) & ~(size_t)255; };
+  size_t o = al(sizeof(int) * ((size_t)nall + 1));
+  if (off_b) *off_b = o;
+  o = al(o + sizeof(int) * (size_t)nall * gather_cap(nnei));
+  if (off_o) *off_o = o;
+  o = al(o + sizeof(int) * slots);
+  if (off_fs) *off_fs = o;
+  return o + sizeof(double) * 3 * slots;
+}
+
+// Where the gathered form takes over: with the atomic virial from 409,600 slots
+// on.  Added / gathered us, Cu lists of 200: atomic virial 1,372 atoms 60 / 62,
+// 2,048 82 / 67, 8,788 257 / 161, 32,000 833 / 380, 131,072 3,560 / 1,336; water
+// of 138: 3,000 atoms 51 / 54, 8,232 109 / 94, 81,000 887 / 480.  Forces alone are
+// added at every size: 500 atoms 27 / 40, 8,788 108 / 139, 32,000 318 / 338, 108,000
+// 1,004 / 1,048 (a lattice whose rows are a multiple of 8 cells puts many atoms'
+// rows on the same memory channels and loses: 131,072 1,323 / 1,227; a
+// contiguous run of centres for each XCD is worse, 1,488).
+static bool gather_pays(int natoms, int nnei, bool atomic_virial) {
+  return atomic_virial && (long long)natoms * nnei >= 409600;
+}
+
 extern "C" size_t dpk_force_virial_gather_workspace_bytes(int natoms, int nnei, int nall) {
   if (natoms < 0 || nnei <= 0 || nall < natoms) return 0;
-  return 256;  // (none is used)
+  if (!gather_pays(natoms, nnei, true)) return 0;
+  return gather_ws_bytes(natoms, nnei, nall, nullptr, nullptr, nullptr);
 }
 
 extern "C" int dpk_force_virial_gather(double* force, double* atom_virial, double* vrow,
@@ -641,13 +827,43 @@ extern "C" int dpk_force_virial_gather(double* force, double* atom_virial, doubl
   DPK_REQUIRE(prec == DPK_PREC_F64 || prec == DPK_PREC_F32 || prec == DPK_PREC_BF16 ||
                   prec == DPK_PREC_F16 || prec == DPK_PREC_F16X2,
               DPK_ERR_ARG, "force_virial_gather: unknown precision %d", prec);
-  DPK_REQUIRE(workspace != nullptr &&
-                  workspace_bytes >= dpk_force_virial_gather_workspace_bytes(natoms, nnei, nall),
-              DPK_ERR_ARG, "force_virial_gather: workspace of %zu bytes", workspace_bytes);
+  const bool gather = gather_pays(natoms, nnei, atom_virial != nullptr);
+  const size_t need = gather ? dpk_force_virial_gather_workspace_bytes(natoms, nnei, nall) : 0;
+  DPK_REQUIRE(need == 0 || (workspace != nullptr && workspace_bytes >= need), DPK_ERR_ARG,
+              "force_virial_gather: workspace %zu < %zu bytes", workspace_bytes, need);
   DPK_REQUIRE((long long)natoms * nnei < (1ll << 31), DPK_ERR_UNSUPPORTED,
               "force_virial_gather: more than 2^31 slots");
   if (nall == 0) return DPK_OK;
   hipStream_t st = as_stream(stream);
+  if (gather) {
+    size_t off_b = 0, off_o = 0, off_fs = 0;
+    gather_ws_bytes(natoms, nnei, nall, &off_b, &off_o, &off_fs);
+    unsigned char* ws = static_cast<unsigned char*>(workspace);
+    int* count = reinterpret_cast<int*>(ws);
+    int* bucket = reinterpret_cast<int*>(ws + off_b);
+    int* ovf = reinterpret_cast<int*>(ws + off_o);
+    double* fs = reinterpret_cast<double*>(ws + off_fs);
+    const int cap = gather_cap(nnei);
+    const long long total = (long long)natoms * nnei;
+    hipLaunchKernelGGL(k_bucket_zero, dim3(cdiv((long long)nall + 1, 256)), dim3(256), 0, st,
+                       count, nall);
+    hipLaunchKernelGGL(k_bucket_fill, dim3(cdiv(total, 256)), dim3(256), 0, st, bucket, count, ovf,
+                       nlist, atype, pair_mask, ntypes, total, nnei, nall, cap);
+    if (prec == DPK_PREC_F64)
+      hipLaunchKernelGGL(k_slot_forces<double>, dim3(cdiv(natoms, 4)), dim3(256), 0, st, fs, force,
+                         vrow, static_cast<const double*>(net_deriv), coord, atype, nlist, std,
+                         natoms, nnei, nall, rcut, rcut_smth, protection, pair_mask, ntypes);
+    else
+      hipLaunchKernelGGL(k_slot_forces<float>, dim3(cdiv(natoms, 4)), dim3(256), 0, st, fs, force,
+                         vrow, static_cast<const float*>(net_deriv), coord, atype, nlist, std,
+                         natoms, nnei, nall, rcut, rcut_smth, protection, pair_mask, ntypes);
+    hipLaunchKernelGGL(k_gather_forces, dim3(cdiv(nall, 4)), dim3(256), 0, st, force, atom_virial,
+                       fs, count, bucket, coord, natoms, nnei, nall, cap);
+    hipLaunchKernelGGL(k_gather_overflow, dim3(64), dim3(256), 0, st, force, atom_virial, fs, count,
+                       ovf, nlist, coord, nnei, nall);
+    DPK_LAUNCHED();
+    return DPK_OK;
+  }
   int rc = zero(force, 3ll * nall, st);
   if (rc == DPK_OK && atom_virial != nullptr) rc = zero(atom_virial, 9ll * nall, st);
   if (rc != DPK_OK || natoms == 0) return rc;

@@ -1044,10 +1044,6 @@ class SeAModel:
         sysd.force = torch.empty((nall, 3), dtype=torch.float64, device=dev)
         sysd.vrow = torch.empty(int(lib.dpk_force_virial_workspace_bytes(nloc)), dtype=torch.uint8,
                                 device=dev)
-        # (dpk_force_virial_gather's workspace)
-        sysd.extra["ws_gather"] = torch.empty(
-            int(lib.dpk_force_virial_gather_workspace_bytes(nloc, S, nall)), dtype=torch.uint8,
-            device=dev)
         sysd.virial = torch.empty((1, 9), dtype=torch.float64, device=dev)
         sysd.energy = torch.empty(1, dtype=torch.float64, device=dev)
         sysd.max_nloc = nloc
@@ -1203,16 +1199,18 @@ class SeAModel:
                 self.fitting.run(s.atom_e, s.gxyz, s.xyz, s.order, s.segments, s.nreal, s.fit,
                                  self.d3, self.axis_neuron, st, xe=s.xe if self.nx else None)
             self._embed_backward(s, st)
-        av = None
+        av = wg = None
         if atomic_virial:
             av = torch.empty((nall, 9), dtype=torch.float64, device=s.force.device)
+            wg = s.extra.get("ws_gather")  # (only the atomic virial needs one)
+            if wg is None:
+                nb = int(lib().dpk_force_virial_gather_workspace_bytes(nloc, self.nnei, nall))
+                wg = s.extra["ws_gather"] = torch.empty(nb, dtype=torch.uint8, device=s.force.device)
         if nloc:
-            # neighbour forces added to the extended atoms' rows
-            wg = s.extra["ws_gather"]
             call("dpk_force_virial_gather", ptr(s.force), ptr(av), ptr(s.vrow), ptr(s.nd),
                  self.prec, ptr(s.coord), ptr(s.atype), ptr(s.nlist), ptr(self.dstd_dev), nloc,
                  self.nnei, nall, self.rcut, self.rcut_smth, self.env_protection,
-                 ptr(self.pair_mask), self.ntypes, ptr(wg), wg.numel(), st)
+                 ptr(self.pair_mask), self.ntypes, ptr(wg), 0 if wg is None else wg.numel(), st)
             call("dpk_frame_sum", ptr(s.virial), ptr(s.vrow), 9, ptr(fs.sums_dev), 1, nloc,
                  ptr(s.ws_fsum), s.ws_fsum.numel(), st)
             call("dpk_frame_sum", ptr(s.energy), ptr(s.atom_e), 1, ptr(fs.sums_dev), 1, nloc,

@@ -672,10 +672,15 @@ int dpk_force_virial_fused(double* force, double* atom_virial, const void* net_d
 /*
  * Forces and virial of an engine's extended region (the MD-engine path:
  * explicit ghosts, nlist [natoms, nnei] of extended-atom indices in
- * [0, nall), coord = the extended coordinates [nall, 3]): one pass over the
- * slots, whose shares are added to their neighbours' rows with FP64 atomics,
- * three consecutive lanes a row.  The workspace is not read or written (its
- * size is a formality of earlier forms).
+ * [0, nall), coord = the extended coordinates [nall, 3]).  Forces alone, and
+ * the atomic virial of few atoms: one pass over the slots, whose shares are
+ * added to their neighbours' rows with FP64 atomics, consecutive lanes a row.
+ * With the atomic virial of many: the slots are binned by neighbour into
+ * fixed-capacity buckets (slots beyond a full bucket are added with atomics at
+ * the end), a first pass writes each slot's neighbour share and the centre's
+ * own force, a second pass sums every extended atom's bucket; this needs the
+ * workspace of dpk_force_virial_gather_workspace_bytes, which is 0 where it is
+ * not used (without atomic_virial the workspace is never looked at).
  * force [nall, 3] and atom_virial [nall, 9] (optional, NULL to skip; the
  * neighbour rows, as dpk_force_virial_fused) are overwritten; vrow
  * [natoms, 9] receives the per-centre virial rows (reduce with

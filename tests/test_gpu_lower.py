@@ -300,12 +300,14 @@ def test_forward_lower_ago_reuse_and_graph_replays(prec):
         m.forward_lower(x1.view(-1, 3)[:-1], ea[:, :-1], None, system=s2, ago=1)
 
 
-def test_forward_lower_bucket_overflow_vs_oracle():
-    """The MD path's neighbour-force gather bins slots into buckets of
-    capacity ~nnei; an atom in more lists than that spills to the overflow
-    list (atomics).  A centre with 100 atoms on a unit shell around it, sel
-    [40]: it is a neighbour of all 100 (capacity 64), forces and atomic
-    virials vs the oracle (1e-10)."""
+@pytest.mark.parametrize("lone", [0, 10200])
+def test_forward_lower_bucket_overflow_vs_oracle(lone):
+    """Forces and atomic virials of the MD path where many slots share one
+    neighbour: a centre with 100 atoms on a unit shell around it, sel [40], is
+    a neighbour of all 100.  Alone they are added to its row; with 10,200 more
+    atoms (no neighbours, 412,040 slots) the slots are gathered from buckets of
+    capacity 64, and the centre's spill to the overflow list.  Against the
+    oracle (1e-10)."""
     from deepmd_amd.model import SeAModel, random_model_dict
     from oracle import geometry, sea
     d = random_model_dict(3, 6.0, 0.5, [40], [8, 16, 32], 16, [16])
@@ -320,6 +322,15 @@ def test_forward_lower_bucket_overflow_vs_oracle():
     a = torch.zeros((1, n), dtype=torch.long)
     ec, ea, mp, nl = geometry.extend_input_and_build_neighbor_list(c, a, m.rcut, m.sel, box=None)
     assert int((nl[0] == 0).sum()) > 64  # the centre sits in more lists than a bucket holds
+    if lone:
+        far = torch.stack(torch.meshgrid(*[torch.arange(22.)] * 3, indexing="ij"), -1)
+        far = 50.0 * (1.0 + far.reshape(-1, 3)[:lone].double())
+        ec = torch.cat([ec.view(1, -1, 3)[:, :n], far[None], ec.view(1, -1, 3)[:, n:]], 1)
+        ec = ec.reshape(1, -1)
+        ea = torch.zeros((1, n + lone), dtype=ea.dtype)
+        nl = torch.cat([nl, torch.full((1, lone, nl.shape[2]), -1, dtype=nl.dtype)], 1)
+        mp = torch.arange(n + lone).view(1, -1)
+        assert n * 40 < 409600 <= (n + lone) * 40
     out = m.forward_lower(ec, ea, nl, mp, do_atomic_virial=True)
     torch.cuda.synchronize()
     ref = sea.forward_lower(om, ec, ea, nl, mp, do_atomic_virial=True)
@@ -327,3 +338,35 @@ def test_forward_lower_bucket_overflow_vs_oracle():
     assert _rel(out["extended_force"].cpu(), ref["extended_force"].detach()) < 1e-10
     assert _rel(out["virial"].cpu(), ref["virial"].detach()) < 1e-10
     assert _rel(out["extended_virial"].cpu(), ref["extended_virial"].detach()) < 1e-10
+
+
+@pytest.mark.parametrize("prec,tol", [("f64", 1e-12), ("f32", 1e-12)])
+def test_forward_lower_gathered_atomic_virial(prec, tol):
+    """Atomic virials of 2,048 atoms and 220 slots (gathered): folded onto the
+    local atoms they are those of the periodic evaluation (cell-blocked
+    atomics), with excluded pairs too; forces are those added without them."""
+    from deepmd_amd import systems
+    from deepmd_amd.model import SeAModel, random_model_dict
+    d = random_model_dict(3, 5.0, 0.5, [110, 110], [8, 16, 32], 4, [16, 16])
+    d["model"]["descriptor"]["exclude_types"] = [[0, 1]]
+    m = SeAModel(d, prec, DEV)
+    x, at, box = systems.fcc(8, 3.6, 0.05, 3)
+    at = np.random.default_rng(1).integers(0, 2, len(at)).astype(np.int32)
+    assert len(at) * 220 >= 409600
+    s = m.system(x[None], at[None], box.reshape(1, 9))
+    ref = m.evaluate(s, atomic_virial=True)
+    ns, nloc = s.fs.frames_host[0].ns, len(at)
+    ext = (s.wrapped.view(1, nloc, 3) + s.fs.shift_vec.view(ns, 1, 3)).reshape(1, -1, 3)
+    ea = s.atype.view(1, nloc).expand(ns, nloc).reshape(1, -1).contiguous()
+    nl = s.nlist.view(1, nloc, -1).clone()
+    own = torch.arange(ns * nloc, device=DEV) % nloc
+    got = m.forward_lower(ext, ea, nl, do_atomic_virial=True)
+    plain = m.forward_lower(ext, ea, nl)
+    near = lambda a, b, tol: _rel(a.cpu(), b.cpu()) <= tol  # noqa: E731
+    fold = lambda v: torch.zeros((nloc, v.shape[-1]), dtype=v.dtype,  # noqa: E731
+                                 device=DEV).index_add_(0, own, v.view(ns * nloc, -1))
+    assert near(got["extended_force"], plain["extended_force"], tol)
+    assert near(fold(got["extended_force"]), ref["force"].view(nloc, 3), tol)
+    av = got["extended_virial"].view(ns * nloc, 9)
+    assert near(fold(av), ref["atom_virial"].view(nloc, 9), tol)
+    assert near(av.sum(0), got["virial"].view(9), 1e-11)
