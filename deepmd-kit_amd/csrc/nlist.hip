@@ -695,11 +695,13 @@ int launch_search_w(const double* wrapped, const int* atype, const int* frame_of
   if (tune(DPK_TUNE_NLIST_MODE) == 1) capb = 0;  // every centre gathers from global memory
   const size_t lds = sizeof(BCand) * (size_t)(capb > 0 ? capb : 1) + wbytes;
   int parts = cell_parts(natoms, ncells, W, ncu);
-  // frames of different sizes: their fullest cells (a small box is one cell)
-  // decide, as far as the other cells' idle workgroups cost little
-  if (ragged && parts < 4) {
-    const int most = 8 * ncu / ncells < 4 ? 8 * ncu / ncells : 4;
-    parts = parts > most ? parts : most;
+  // cells above the mean decide, so four where that leaves no CU with two of them
+  // (27 and 54 cells of 38 atoms: 84 us with three, 64 with four); frames that
+  // differ, whose fullest cells are far above it (a small box is one cell), as far
+  // as the other cells' idle workgroups cost little
+  if (parts < 4) {
+    const int most = (ragged ? 8 : 1) * ncu / ncells;
+    if (ragged || most >= 4) parts = most < parts ? parts : (most < 4 ? most : 4);
   }
   hipLaunchKernelGGL((k_search_cells<MAXC, W>), dim3(ncells * parts), dim3(64 * W), lds, st,
                      wrapped, atype, frame_of, frames, atom_cell, cell_start, cell_atoms, img_pos,
@@ -713,9 +715,11 @@ int launch_search_w(const double* wrapped, const int* atype, const int* frame_of
 // and hide the latency of the per-centre scan and sort (a workgroup of 16
 // takes a whole CU); fewer where cells hold few atoms (measured: 24 atoms a
 // cell, 12,288 in all, 8 wavefronts 68 us, 16 84; 32 a cell, 3,993 in all, 90
-// and 64).  Batches of frames take 16 from 8 atoms a cell on: their cells
-// differ, and the fullest -- a frame of one cell -- are the longest (96 frames
-// of 24..768 atoms: 4 wavefronts and 1.25x staged 534 us, 16 and 3x 291).
+// and 64).  Batches of frames that differ (`ragged`) take 16 from 8 atoms a cell
+// on: the fullest cells -- a frame of one cell -- are the longest (96 frames of
+// 24..768 atoms: 4 wavefronts and 1.25x staged 534 us, 16 and 3x 291).  Frames of
+// one size must not: 4 x 3,000 water atoms 89 -> 279 us, 128 x 192 145 -> 281, 4 x
+// 8,788 Cu atoms 260 -> 358 with that treatment.
 template <int MAXC>
 int launch_search(const double* wrapped, const int* atype, const int* frame_of,
                   const dpk_frame* frames, const int* atom_cell, const int* cell_start,
@@ -972,10 +976,13 @@ extern "C" int dpk_nlist_build(int* nlist, double* coord_wrapped, int* status_de
   hipLaunchKernelGGL(k_rank, dim3(cdiv(natoms, 256)), dim3(256), 0, st, atom_cell, cell_start,
                      w.cell_tmp, natoms, atom_slot, cell_atoms);
   DPK_LAUNCHED();
+  // frames of one size have a whole share of the atoms and of the cells each (a
+  // batch that differs and still divides evenly only misses its own treatment)
+  const bool ragged = natoms % nframes != 0 || ncells % nframes != 0;
 #define DPK_SEARCH(M)                                                                       \
   return launch_search<M>(coord_wrapped, atype, frame_of, frames, atom_cell, cell_start,   \
                           cell_atoms, img_pos, shift_vec, rcut, si, natoms, ncells, nlist, \
-                          status_dev, nframes > 1, st)
+                          status_dev, ragged, st)
   if (max_cand <= 256) DPK_SEARCH(256);
   if (max_cand <= 512) DPK_SEARCH(512);
   if (max_cand <= 1024) DPK_SEARCH(1024);

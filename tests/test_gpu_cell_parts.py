@@ -25,6 +25,8 @@ def _frame(n, edge, seed):
     [(1, 5.0)], [(16, 7.0)], [(17, 7.0)], [(81, 9.3)], [(130, 9.9)],       # one cell
     [(400, 16.0)], [(1000, 21.0)],                                       # 27 and 64 cells
     [(24, 7.2), (43, 7.0), (90, 11.0), (300, 17.0), (7, 6.0)],           # one batch
+    [(81, 9.3)] * 4, [(192, 12.4)] * 33,                                 # frames of one size
+    [(400, 16.0)] * 12, [(60, 9.0), (100, 9.5), (80, 9.2)],              # (the last divides too)
 ])
 def test_shared_cells(sizes):
     d = random_model_dict(3, 5.0, 0.5, [60, 60], [25, 50, 100], 16, [32, 32])
