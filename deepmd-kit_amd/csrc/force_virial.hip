@@ -303,12 +303,15 @@ __global__ void __launch_bounds__(64 * W) k_force_cells(
     const int* __restrict__ cell_start, const int* __restrict__ cell_atoms,
     const int* __restrict__ atom_cell, const int* __restrict__ atom_slot, int nnei, double rcut,
     double rcut_smth, double protection, const int* __restrict__ pair_mask, int ntypes,
-    int parts) {
+    int ncells, int share, int full, int most) {
   __shared__ double tab[kCellTab * 3];
-  // `parts` workgroups share a cell's centres, W at a time in turn
-  const int cell = blockIdx.x / parts, first = (blockIdx.x % parts) * W;
+  // `share` workgroups take a cell's centres, W at a time in turn, `most` those
+  // of a cell of more than `full`; the cells' first workgroups start first, those
+  // that find nothing to do last
+  const int cell = blockIdx.x % ncells, part = blockIdx.x / ncells, first = part * W;
   const int a0 = cell_start[cell], a1 = cell_start[cell + 1];
-  if (a1 <= a0 + first) return;  // uniform over the workgroup
+  const int parts = a1 - a0 > full ? most : share;
+  if (part >= parts || a1 <= a0 + first) return;  // uniform over the workgroup
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   for (int q = threadIdx.x; q < kCellTab * 3; q += blockDim.x) tab[q] = 0.0;
   const dpk_frame& fd = frames[frame_of[cell_atoms[a0]]];
@@ -962,13 +965,21 @@ extern "C" int dpk_force_virial_cells(double* force, double* atom_virial, const 
   int dev = 0, ncu = 0;
   DPK_HIP(hipGetDevice(&dev));
   DPK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  const int parts = cell_parts(natoms, ncells, nw, 3 * ncu);  // three tables fit a CU's LDS
+  // Workgroups a cell: three tables fit a CU's LDS, but a second and third
+  // workgroup clears and adds a table of its own, so an ordinary cell has as many
+  // as give half of that, and one of more than twice the mean (frames that differ)
+  // all.  343 cells of 24 atoms: one workgroup 43 us, two 50; 256 of 32: 42, three 47;
+  // 216 of 76: 187, three 216; 125 of 70: three 97, six 107, one 112; 313 cells of
+  // 96 frames of up to 100 atoms: one 123, two 81.
+  const int share = cell_parts(natoms, ncells, nw, 3 * ncu / 2);
+  const int most = cell_parts(natoms, ncells, nw, 3 * ncu);
+  const int full = (int)(2ll * natoms / ncells);
 #define DPK_FORCE_CELLS(GT, NW)                                                              \
-  hipLaunchKernelGGL((k_force_cells<GT, NW>), dim3(ncells * parts), dim3(64 * NW), 0, st, force, vrow, \
+  hipLaunchKernelGGL((k_force_cells<GT, NW>), dim3(ncells * most), dim3(64 * NW), 0, st, force, vrow, \
                      atom_virial, static_cast<const GT*>(net_deriv), coord_wrapped, atype,     \
                      frame_of, frames, nlist, shift_vec, img_shift, std, w.cell_start,         \
                      w.cell_atoms, w.atom_cell, w.atom_slot, nnei, rcut, rcut_smth,             \
-                     protection, pair_mask, ntypes, parts)
+                     protection, pair_mask, ntypes, ncells, share, full, most)
 #define DPK_FORCE_CELLS_W(GT)            \
   if (nw == 16) DPK_FORCE_CELLS(GT, 16); \
   else if (nw == 8) DPK_FORCE_CELLS(GT, 8); \
