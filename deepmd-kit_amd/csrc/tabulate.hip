@@ -8,7 +8,9 @@
 // remaining slots, weight nnei - j), :234-341 (grad), :343-447 (grad_grad).
 //
 // Four basis functions (the se_a env matrix, op and fused model alike): one
-// wavefront an atom, channels on the lanes, see k_tab4_fwd / k_tab4_bwd below.
+// wavefront an atom (several in the backward where atoms are few), channels on
+// the lanes, see k_tab4_fwd / k_tab4_bwd below; the backward of narrow nets puts
+// the slots there (k_tab4_bwd_narrow).
 // Other basis dimensions (9, 16, 25) and grad_grad: one workgroup an atom;
 // forward and grad_grad put the L channels on the threads and walk the
 // neighbours, grad puts the neighbours on the threads and walks the channels,
@@ -212,9 +214,12 @@ struct TabSet {
 // is taken in their order by one lane a channel; the backward's five sums over
 // the channels are folded across the lanes for four slots together.
 // Measured at 12,288 x 92 x 100, FP32: forward 207 -> 119 us (17 TB/s of
-// table), backward 202 -> 151; 1,001 x 46 x 100, FP64: 30 -> 18 and 23 -> 23.
-// What bounds them now is the L2 bandwidth of the rows: spreading an atom over
-// four wavefronts changes nothing at any size (1,001 atoms: 18.1 and 18.3 us).
+// table), backward 202 -> 151.  What bounds them now is the L2 bandwidth of the
+// rows, and below some thousand atoms a wavefront's own pace: the forward gives
+// channels beyond 64 CPL to other workgroups (100 x 92 slots of 256: 47 -> 28 us),
+// the backward, whose slots don't meet, shares an atom (tab_split).  Spreading an
+// atom's slots in the forward, whose sums then meet, gains nothing (1,001 atoms:
+// 18.1 and 18.3 us).
 template <typename T>
 struct Tab4 {
   const T* em;        // [natoms, nnei, 4]
@@ -227,6 +232,7 @@ struct Tab4 {
   T* dx;              // backward: d em_x [natoms, nnei], or null: added to d em[..., 0]
   T scale;
   int natoms, nnei, L;
+  int lp;             // backward: log2 of the wavefronts an atom
   TabSet<T> ts;
 };
 
@@ -290,7 +296,8 @@ __global__ void __launch_bounds__(256) k_tab4_fwd(Tab4<T> A) {
   tc = __builtin_amdgcn_readfirstlane(tc < 0 ? 0 : tc);
   const T* ea = A.em + (size_t)atom * A.nnei * 4;
   const int L = A.L;
-  for (int kc = 0; kc < L; kc += 64 * CPL) {
+  // (each of the grid's rows of workgroups takes a run of 64 CPL channels)
+  for (int kc = blockIdx.y * 64 * CPL; kc < L; kc += gridDim.y * 64 * CPL) {
     const int k0 = kc + lane * CPL;
     const int kl = k0 < L ? k0 : 0;
     T acc[CPL][4];
@@ -408,12 +415,15 @@ __device__ __forceinline__ T sum4(T v0, T v1, T v2, T v3) {
 template <typename T, int CPL, bool VEC, bool ONE>
 __global__ void __launch_bounds__(256) k_tab4_bwd(Tab4<T> A) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int atom = blockIdx.x * 4 + wave;
+  // 1 << lp wavefronts share an atom: each takes every (1 << lp)-th four slots
+  const int unit = blockIdx.x * 4 + wave, atom = unit >> A.lp, mask = (1 << A.lp) - 1,
+            part = unit & mask;
   if (atom >= A.natoms) return;
   int tc = A.atype != nullptr ? A.atype[atom] : 0;
   tc = __builtin_amdgcn_readfirstlane(tc < 0 ? 0 : tc);
   const T* ea = A.em + (size_t)atom * A.nnei * 4;
   const int L = A.L, row = lane >> 4, c = lane & 15;
+  int turn = 0;  // fours of the chunks before
   T dy[CPL][4];
   auto load_dy = [&](int k0) {
 #pragma unroll
@@ -440,7 +450,9 @@ __global__ void __launch_bounds__(256) k_tab4_bwd(Tab4<T> A) {
     int c0 = 0;
     for (; c0 < nb && !s.stop; c0 += 64) {
       s.take(A, ti, e, ex, last, c0, nb, lane);
-      for (int j = 0; j < s.cnt; j += 4) {
+      const int first = (part - turn) & mask;
+      turn += (s.cnt + 3) / 4;
+      for (int j = 4 * first; j < s.cnt; j += 4 << A.lp) {
         T v[4][5];
 #pragma unroll
         for (int u = 0; u < 4; ++u)
@@ -494,26 +506,117 @@ __global__ void __launch_bounds__(256) k_tab4_bwd(Tab4<T> A) {
         }
       }
       if (s.stop) {  // the slots that the fold stands for
-        const int z = c0 + s.cnt;
-        for (int q = 4 * z + lane; q < 4 * nb; q += 64) od[q] = T(0);
+        const int z = c0 + s.cnt, q0 = lane + 64 * part, step = 64 << A.lp;
+        for (int q = 4 * z + q0; q < 4 * nb; q += step) od[q] = T(0);
         if (ox != nullptr)
-          for (int q = z + lane; q < nb; q += 64) ox[q] = T(0);
+          for (int q = z + q0; q < nb; q += step) ox[q] = T(0);
       }
     }
   }
+}
+
+// Backward of narrow nets: a slot a lane, the channels in turn, dy in LDS; one
+// workgroup an atom: up to 16 channels, and 32 where the slots fill a wavefront.
+// (Channels on the lanes leave half of them idle and fold every slot's sums across
+// all: 12,288 x 92 slots of 8 / 16 / 32 / 48 channels in FP32 114 us each, this 27 /
+// 51 / 92 / 130; 20 slots of 32 channels 31, this 41.)
+constexpr int kNarrow = 32;
+
+template <typename T>
+__global__ void __launch_bounds__(128) k_tab4_bwd_narrow(Tab4<T> A) {
+  __shared__ __align__(4 * sizeof(T)) T dys[kNarrow][4];
+  __shared__ int first[kMaxTabTypes];
+  const int atom = blockIdx.x, L = A.L;
+  int tc = A.atype != nullptr ? A.atype[atom] : 0;
+  tc = tc < 0 ? 0 : tc;
+  const T* ea = A.em + (size_t)atom * A.nnei * 4;
+  const T* xa = A.emx != nullptr ? A.emx + (size_t)atom * A.nnei : nullptr;
+  for (int q = threadIdx.x; q < 4 * L; q += blockDim.x)
+    dys[q % L][q / L] = A.dy[(size_t)atom * 4 * L + q] * A.scale;
+  if (threadIdx.x < (unsigned)A.ts.ntypes) first[threadIdx.x] = A.nnei;
+  __syncthreads();
+  for (int t = 0; t < A.ts.ntypes; ++t) {  // the blocks' folds
+    const int b0 = A.ts.sec[t], b1 = A.ts.sec[t + 1];
+    if (b1 <= b0) continue;
+    const T last = xa != nullptr ? xa[b1 - 1] : ea[(size_t)(b1 - 1) * 4];
+    for (int j = b0 + threadIdx.x; j < b1; j += blockDim.x) {
+      const T* r = ea + (size_t)j * 4;
+      if ((xa != nullptr ? xa[j] : r[0]) == last && r[1] == T(0) && r[2] == T(0) && r[3] == T(0))
+        atomicMin(&first[t], j);
+    }
+  }
+  __syncthreads();
+  for (int t = 0; t < A.ts.ntypes; ++t) {
+    const int b0 = A.ts.sec[t], b1 = A.ts.sec[t + 1];
+    if (b1 <= b0) continue;
+    const int net = A.net_of != nullptr ? A.net_of[tc * A.ts.ntypes + t] : 0;
+    const TabInfo<T>& ti = A.ts.ti[net];
+    const T* tab = A.tables + A.ts.off[net];
+    for (int j = b0 + threadIdx.x; j < b1; j += blockDim.x) {
+      const T* r = ea + (size_t)j * 4;
+      T gx = T(0), gm[4] = {T(0), T(0), T(0), T(0)};
+      if (j <= first[t]) {
+        int idx;
+        T x, ext;
+        locate<T>(ti, xa != nullptr ? xa[j] : r[0], idx, x, ext);
+        const T* row = tab + (size_t)idx * L * 6;
+        const T r0 = r[0], r1 = r[1], r2 = r[2], r3 = r[3];
+#pragma clang loop unroll_count(sizeof(T) == 4 ? 2 : 1)
+        for (int k = 0; k < L; ++k) {
+          T val, grd;
+          piece<T>(row + 6 * k, x, ext, val, grd);
+          const T d0 = dys[k][0], d1 = dys[k][1], d2 = dys[k][2], d3 = dys[k][3];
+          gx += grd * (r0 * d0 + r1 * d1 + r2 * d2 + r3 * d3);
+          gm[0] += val * d0;
+          gm[1] += val * d1;
+          gm[2] += val * d2;
+          gm[3] += val * d3;
+        }
+        const T w = j == first[t] ? T(b1 - j) : T(1);
+        gx *= w;
+        for (int m = 0; m < 4; ++m) gm[m] *= w;
+      }
+      const size_t s = (size_t)atom * A.nnei + j;
+      if (A.dx != nullptr) A.dx[s] = gx;
+      else gm[0] += gx;
+      for (int m = 0; m < 4; ++m) A.out[s * 4 + m] = gm[m];
+    }
+  }
+}
+
+// Wavefronts an atom of the backward (log2): several, of eight slots and more
+// each, while they fit the chip together (16 a CU).  FP32, 100 channels, with 1 / 2
+// / 4 / 8 us: 100 atoms of 200 slots 59 / 35 / 23 / 16, 1,001 of 92 33 / 25 / 22 /
+// 24, of 200 61 / 44 / 40 / 42, 12,288 of 92 151 / 153 / 164 / 207.
+inline int tab_split(int natoms, int nnei, int ncu) {
+  int lp = 0;
+  while (lp < 3 && (2l << lp) * natoms <= 16l * ncu && (16 << lp) <= nnei) ++lp;
+  return lp;
 }
 
 // Channels a lane: two for wide nets (16-byte loads, lanes filled), one where
 // 64 lanes hold all of them, or where L is odd (the rows are then aligned to
 // one channel only).  Tables that are not aligned are read value by value.
 template <typename T>
-int launch_tab4(bool fwd, const Tab4<T>& A, hipStream_t st) {
+int launch_tab4(bool fwd, Tab4<T>& A, hipStream_t st) {
   if (A.natoms == 0) return DPK_OK;
-  const dim3 g(cdiv(A.natoms, 4)), b(256);
+  const dim3 b(256);
   const size_t at = reinterpret_cast<size_t>(A.tables);
+  if (!fwd && (A.L <= 16 || (A.L <= kNarrow && A.nnei >= 64))) {
+    hipLaunchKernelGGL((k_tab4_bwd_narrow<T>), dim3(A.natoms), dim3(A.nnei >= 128 ? 128 : 64), 0,
+                       st, A);
+    DPK_LAUNCHED();
+    return DPK_OK;
+  }
+  int dev = 0, ncu = 0;
+  DPK_HIP(hipGetDevice(&dev));
+  DPK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  A.lp = fwd ? 0 : tab_split(A.natoms, A.nnei, ncu);
+  const dim3 g(cdiv((long long)A.natoms << A.lp, 4));
 #define DPK_TAB4(CPL, VEC)                                                                 \
   do {                                                                                     \
-    if (fwd) hipLaunchKernelGGL((k_tab4_fwd<T, CPL, VEC>), g, b, 0, st, A);                  \
+    if (fwd)                                                                               \
+      hipLaunchKernelGGL((k_tab4_fwd<T, CPL, VEC>), dim3(g.x, cdiv(A.L, 64 * CPL)), b, 0, st, A); \
     else if (A.L <= 64 * CPL)                                                              \
       hipLaunchKernelGGL((k_tab4_bwd<T, CPL, VEC, true>), g, b, 0, st, A);                   \
     else hipLaunchKernelGGL((k_tab4_bwd<T, CPL, VEC, false>), g, b, 0, st, A);               \
