@@ -9,17 +9,21 @@
 //             g_z_{l-1} = g_y_{l-1} sd_{l-1}
 //   dE/dD = g_z_1 W_1^T
 // Rows are slots (atoms grouped by type); a tile belongs to one type and takes
-// that type's weights, so a step of two types and three layers is 10 launches
-// instead of 31.
+// that type's weights, so a step of three layers is 9 launches whatever the
+// number of types (three products forward, the energy, three back, and the
+// descriptor's two) instead of 31 with two.
 //
 // What bounds it: with few atoms the launches and the length of the sum over
-// K, else the FP64 pipe (64 cycles a v_mfma_f64_16x16x4).  Both operands come straight from memory into registers, four steps
-// of eight K values ahead: W is laid out once in the order the lanes read it
-// (dpk.h), and a lane's two K values of A are adjacent.
+// K, else the FP64 pipe (64 cycles a v_mfma_f64_16x16x4).  Both operands come
+// straight from memory into registers, four steps of eight K values ahead: W is
+// laid out once in the order the lanes read it (dpk.h), and a lane's two K values
+// of A are adjacent.
 // Measured, fitting kernels of a step (descriptor apart), against hipBLASLt
 // products and elementwise kernels a type: water of 81 atoms 266 -> 43 us, of
 // 1,536 atoms 255 -> 127; Cu of 5,324 atoms 380 -> 372 (one type: 12 launches
-// -> 7).  FP32 stays with the library: there this kernel took 559 us against
+// -> 7).  With many rows of wide layers the library's products are faster (Cu of
+// 13,500 atoms 1,081 against 986, 131,072 9,509 against 8,391): the model calls
+// this up to the rows of Fitting.chain_rows.  FP32 stays with the library: there this kernel took 559 us against
 // 591 at 12,288 atoms and 1972 against 1290 at 37,700.
 #include "dpk_common.h"
 #include "tanh64.h"

@@ -11,7 +11,7 @@ hand-written adjoint kernels:
     embedding + R^T G      -> dpk_embed_fwd          (MFMA)
     G^T R R^T G            -> dpk_fit_descriptor_fwd (rows grouped by type)
     fitting net (+ grad)   -> hipBLASLt GEMMs + dpk_fit_layer_fwd / _bwd, dpk_fit_energy
-                              (FP64: dpk_fit_chain_f64; split FP16: dpk_fit_l1_*, dpk_fit_tail_*)
+                              (FP64, few rows: dpk_fit_chain_f64; split FP16: dpk_fit_l1_*, dpk_fit_tail_*)
     dE/dxyz                -> dpk_fit_descriptor_bwd
     dE/d em (recompute)    -> dpk_embed_bwd          (MFMA)
     forces, virial         -> dpk_force_virial_cells + dpk_frame_sum
@@ -333,7 +333,8 @@ class Fitting:
     dpk_fit_descriptor_fwd / _bwd.  Hidden layers: tanh, optional idt, resnet
     0 / 1 / 2; output layer: linear to one value (the reference's
     EnergyFittingNet, network.py:935-1006).  FP64 tanh nets of widths
-    divisible by 16 run as a whole in one call (dpk_fit_chain_f64).  16-bit (BF16 /
+    divisible by 16 run as a whole in one call (dpk_fit_chain_f64) up to the
+    rows of chain_rows.  16-bit (BF16 /
     FP16) nets of 2
     or 3 hidden layers of (padded) width 256 run layers 2..L, the energy and
     the backward down to dE/dz_1 in one kernel (dpk_fit_tail_bf16 / _f16)
@@ -351,8 +352,20 @@ class Fitting:
     # split FP16: descriptor + layer 1 (and their backward) in one kernel each
     # (dpk_fit_l1_fwd / _bwd) instead of writing D and dE/dD around two GEMMs
     FUSED_L1 = True
-    # FP64 tanh nets: the whole fitting in one call (dpk_fit_chain_f64)
+    # FP64 tanh nets: the whole fitting in one call (dpk_fit_chain_f64), up to
+    # chain_rows rows a type
     CHAIN = True
+
+    @staticmethod
+    def chain_rows(width: int) -> float:
+        """Rows a type up to which dpk_fit_chain_f64 is the faster form for
+        layers of at most ``width``: its launches are few, the library's tiles
+        larger.  Time over the library's (d3 m2 = 2048; rows a type): width 64
+        0.73 at 1,372, 0.92 at 42,592; 128 0.80 at 1,372, 0.98 at 10,976, 1.08 at
+        42,592; 256 0.89 at 1,372, 0.97 at 5,324, 1.08 at 6,912 (two types 0.93 at
+        5,488, 1.02 at 6,750); 512 0.92 at 1,372, 1.04 at 2,048; 1024 0.65 at 256,
+        1.02 at 500."""
+        return float("inf") if width <= 64 else min(11000.0, 3.6e8 / width ** 2)
 
     def __init__(self, nets, bias_atom_e, out_bias, prec: str, device, nx: int = 0):
         self.prec = prec
@@ -509,7 +522,7 @@ class Fitting:
                     "D": torch.empty((nd, 2 * self.din), dtype=gd, device=dev),
                     "GD": torch.empty((nd, self.din), dtype=torch.float32, device=dev),
                     "cx": None}
-        if self.chain is not None:
+        if self.chain is not None and n <= len(self.nets) * self.chain_rows(hmax):
             nb = int(lib().dpk_fit_chain_f64_workspace_bytes(n, nl, self.chain["widths"][1]))
             return {"D": torch.empty((n, self.din), dtype=gd, device=dev),
                     "ws": torch.empty(max(nb, 1), dtype=torch.uint8, device=dev)}
@@ -551,7 +564,7 @@ class Fitting:
         pc = self.prec_code
         if self.nx and xe is None:
             raise ValueError("the fitting nets take frame / atomic parameters: xe is required")
-        if self.chain is not None:
+        if "ws" in bf:  # (buffers chose the form)
             ch = self.chain
             segs = ctypes_int_array([v for seg in segments for v in seg])
             call("dpk_fit_chain_f64", ch["L"], ch["widths"][1], ch["res"][1], ch["params"][1],

@@ -23,16 +23,20 @@ def _torch_energy(layers, d):
     return (x @ torch.tensor(layers[-1].w))[:, 0] + float(layers[-1].b[0])
 
 
-@pytest.mark.parametrize("widths,d3,m2,rows,dt", [
-    ([240, 240, 240], 100, 16, [27, 54], True),      # 16 x 16 tiles, K split
-    ([240, 240, 240], 100, 16, [513, 1000], True),   # 32 x 32 tiles
-    ([240, 240], 128, 16, [5000], False),            # 64 x 64 tiles
-    ([32, 64, 64], 64, 4, [1, 0, 17], True),         # resnet 2 and 1, an empty type
-    ([16], 32, 8, [33], False),                      # one layer
-    ([48, 48, 96], 40, 16, [16, 15, 2], True),
-    ([256, 256, 256], 128, 16, [64, 65], False),
+@pytest.mark.parametrize("widths,d3,m2,rows,dt,chain", [
+    ([240, 240, 240], 100, 16, [27, 54], True, True),      # 16 x 16 tiles, K split
+    ([240, 240, 240], 100, 16, [513, 1000], True, True),   # 32 x 32 tiles
+    ([240, 240], 128, 16, [5000], False, True),            # 64 x 64 tiles
+    ([32, 64, 64], 64, 4, [1, 0, 17], True, True),         # resnet 2 and 1, an empty type
+    ([16], 32, 8, [33], False, True),                      # one layer
+    ([48, 48, 96], 40, 16, [16, 15, 2], True, True),
+    ([256, 256, 256], 128, 16, [64, 65], False, True),
+    ([240, 240], 32, 4, [5493], True, True),               # the line of width 256
+    ([240, 240], 32, 4, [5494], True, False),              # beyond: the library's products
+    ([512, 512], 32, 4, [1300, 1500], False, False),
+    ([64, 64], 24, 4, [12000], True, True),
 ])
-def test_fit_chain_vs_autograd(widths, d3, m2, rows, dt):
+def test_fit_chain_vs_autograd(widths, d3, m2, rows, dt, chain):
     rng = np.random.default_rng(5)
     nt = len(rows)
     nets = [M._layers(M._rand_net(rng, [d3 * m2] + widths + [1], dt, True)) for _ in range(nt)]
@@ -46,7 +50,9 @@ def test_fit_chain_vs_autograd(widths, d3, m2, rows, dt):
     x = torch.tensor(xyz, device=DEV)
     ae = torch.full((n,), float("nan"), dtype=torch.float64, device=DEV)
     gx = torch.full((n, 4, d3), float("nan"), dtype=torch.float64, device=DEV)
-    fit.run(ae, gx, x, torch.tensor(order, device=DEV), segs, n, fit.buffers(n), d3, m2,
+    bf = fit.buffers(n)
+    assert ("ws" in bf) == chain
+    fit.run(ae, gx, x, torch.tensor(order, device=DEV), segs, n, bf, d3, m2,
             torch.cuda.current_stream().cuda_stream)
     torch.cuda.synchronize()
     ref = torch.tensor(xyz, requires_grad=True)
