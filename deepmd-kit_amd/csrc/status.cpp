@@ -26,7 +26,7 @@ static std::atomic<int> g_tune[DPK_TUNE_COUNT] = {
     {0},    // DPK_TUNE_NLIST_MODE: 0 staged cell neighbourhoods, 1 per-centre gather
     {125},  // DPK_TUNE_NLIST_STAGE_PCT: staging capacity, % of the mean neighbourhood
     {0},    // DPK_TUNE_FORCE_MODE: 0 cell-blocked, 1 per-atom
-    {100},  // DPK_TUNE_EMBED_GRID_PCT: persistent BF16 embedding grid, % of resident slots
+    {100},  // DPK_TUNE_EMBED_GRID_PCT: persistent 16-bit embedding grid, % of the default
     {0},    // DPK_TUNE_NLIST_WAVES: search wavefronts per cell workgroup (0 = from the density)
     {0},    // DPK_TUNE_FORCE_WAVES: cell-blocked force wavefronts per workgroup (0 = auto)
     {0},    // DPK_TUNE_NLIST_SORT: 0 packed keys + full-key fallback, 1 full keys only

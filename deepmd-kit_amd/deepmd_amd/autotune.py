@@ -4,7 +4,7 @@ The kernels have equivalent organisations whose speed depends on the system
 (atoms per cell, neighbour count, number of atoms vs the device's resident
 wavefronts): the neighbour search with or without the cell neighbourhood
 staged in LDS and its staging capacity, the cell-blocked or per-atom force
-kernel, and the size of the persistent BF16 embedding grid.  ``autotune``
+kernel, and the size of the persistent 16-bit embedding grid.  ``autotune``
 times whole E+F+V steps of a real system for each candidate value (HIP
 events on the launch stream), one tunable at a time, keeps the fastest and
 leaves it in the model's own tuning set (``model.tuning``, made current

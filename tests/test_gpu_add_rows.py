@@ -27,10 +27,13 @@ def test_force_virial_rows(nf, nloc, nall, nnei):
     # entries outside the region add nothing to any row
     out = np.where(rng.random(nl.shape) < 0.1, nall + 3, nl).astype(np.int32)
     v2, av2 = torch.ops.deepmd.prod_virial_se_a(to(nd), to(ed), to(rij), to(out), nloc, nall)
+    f2 = torch.ops.deepmd.prod_force_se_a(to(nd), to(ed), to(out), nloc, nall)
     rv, rav = cops.prod_virial_a(nd, ed, rij, nl, nall)
     rv2, rav2 = cops.prod_virial_a(nd, ed, rij, np.where(out >= nall, -1, out), nall)
     rf = cops.prod_force_a(nd, ed, nl, nall)
+    # (the centre's own row takes every slot's share, listed neighbour or not)
+    rf2 = cops.prod_force_a(nd, ed, np.where(out >= nall, -1, out), nall)
     # sums of at most nloc nnei products rounded at 1.1e-16
-    for got, ref in ((f, rf), (v, rv), (av, rav), (v2, rv2), (av2, rav2)):
+    for got, ref in ((f, rf), (f2, rf2), (v, rv), (av, rav), (v2, rv2), (av2, rav2)):
         ref = ref.reshape(got.shape)
         assert np.max(np.abs(got.cpu().numpy() - ref)) <= 1e-13 * max(np.max(np.abs(ref)), 1.0)

@@ -147,3 +147,29 @@ def test_embed_f16x2_operand_bits(neuron, scale, natoms):
         err += [float((g.cpu().double() - r).norm() / r.norm()) for g, r in pairs]
     print(f"{neuron} x {scale} n={natoms}: " + " ".join(f"{v:.2e}" for v in err), flush=True)
     assert all(v < t for v, t in zip(err, SMALL[neuron, scale])), err
+
+
+@pytest.mark.parametrize("natoms", [40, 700, 1700])  # four, two and one wavefronts an atom
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_embed_f16x2_not_finite(natoms, bad):
+    """A row that is not finite stays in its atom: the others' results are what
+    they are without it, bit for bit."""
+    d, at, em, nl, gx = _case([25, 50, 100], [20, 33], True, natoms, False)
+    nl[4, 0] = 0
+    m = SeAModel(d, "f16x2", DEV)
+    to = lambda a: torch.tensor(a, device=DEV).contiguous()  # noqa: E731
+    out = []
+    for v in (em[4, 0, 0], bad):
+        em[4, 0, 0] = v
+        s = SimpleNamespace(fs=SimpleNamespace(natoms=natoms), em=to(em), atype=to(at),
+                            nlist=to(nl), gxyz=to(gx), nd=torch.zeros(*em.shape, device=DEV),
+                            xyz=torch.zeros(natoms, 4, m.d3, device=DEV))
+        st = torch.cuda.current_stream().cuda_stream
+        m._embed_forward(s, st)
+        m._embed_backward(s, st)
+        torch.cuda.synchronize()
+        out.append((s.xyz.cpu().numpy(), s.nd.cpu().numpy()))
+    keep = np.arange(natoms) != 4
+    for a, b in zip(*out):
+        assert np.array_equal(a[keep], b[keep])
+    assert not np.isfinite(out[1][0][4]).all() and not np.isfinite(out[1][1][4, 0]).all()

@@ -71,3 +71,33 @@ def test_fit_chain_vs_autograd(widths, d3, m2, rows, dt, chain):
         err = float((got.cpu() - want).abs().max() / want.abs().max())
         print(f"{name} {widths} {rows}: {err:.2e}", flush=True)
         assert err < 1e-12, name
+
+
+@pytest.mark.parametrize("rows", [[20, 30], [700, 1400]])  # K split over the wavefronts, 32 x 32
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_fit_chain_not_finite(rows, bad):
+    """A slot that is not finite stays alone: the others' energies and gradients
+    are what they are without it, bit for bit."""
+    rng = np.random.default_rng(6)
+    nets = [M._layers(M._rand_net(rng, [100 * 16, 240, 240, 1], True, True)) for _ in rows]
+    fit = M.Fitting(nets, np.zeros(2), np.zeros(2), "f64", torch.device(DEV))
+    n = sum(rows)
+    segs = [(0, 0, rows[0]), (1, rows[0], n)]
+    order = torch.arange(n, dtype=torch.int32, device=DEV)
+    xyz = rng.normal(size=(n, 4, 100)) * 0.3
+    at = rows[0] - 1  # the last row of a type, which tiles beyond the end read again
+    out = []
+    for v in (xyz[at, 1, 3], bad):
+        xyz[at, 1, 3] = v
+        ae = torch.zeros(n, dtype=torch.float64, device=DEV)
+        gx = torch.zeros((n, 4, 100), dtype=torch.float64, device=DEV)
+        bf = fit.buffers(n)
+        assert "ws" in bf
+        fit.run(ae, gx, torch.tensor(xyz, device=DEV), order, segs, n, bf, 100, 16,
+                torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        out.append((ae.cpu().numpy(), gx.cpu().numpy()))
+    keep = np.arange(n) != at
+    for a, b in zip(*out):
+        assert np.array_equal(a[keep], b[keep])
+    assert not np.isfinite(out[1][1][at]).all()
