@@ -45,6 +45,9 @@ int tune(int key);  // current value of a DPK_TUNE_* tunable
     }                                                                       \
   } while (0)
 
+// Current device and its CUs; the CUs are asked for once a device (status.cpp).
+int device_cus(int* dev, int* ncu);
+
 inline hipStream_t as_stream(dpk_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 
 inline unsigned int cdiv(long long a, long long b) { return (unsigned int)((a + b - 1) / b); }

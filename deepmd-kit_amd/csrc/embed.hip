@@ -33,6 +33,7 @@
 // / FP16 (FP32 accumulate, FP32 activations) have their own kernels in
 // namespace bf (LDS-resident weights, K = 32 MFMA); FP16X2 is in
 // embed_f16x2.hip, FP64 in embed_f64.hip.
+#include <atomic>
 #include <type_traits>
 
 #include "dpk_common.h"
@@ -833,20 +834,22 @@ int launch(bool fwd, void* out, const void* em, const void* gx, const int* atype
   const size_t lds = RESIDENT ? (size_t)nnets * NET_BYTES : 0;
   // resident workgroups per device, cached per (device, direction, variant, nnets)
   constexpr int kDev = 64, kRes = kResidentMaxBytes / NET_BYTES + 1;
-  static int cache[kDev][2][8][kRes];  // one per format E
-  int dev = 0;
-  DPK_HIP(hipGetDevice(&dev));
+  static std::atomic<int> cache[kDev][2][8][kRes];  // one per format E
+  int dev = 0, ncu = 0;
+  const int rc = device_cus(&dev, &ncu);
+  if (rc != DPK_OK) return rc;
   DPK_REQUIRE(dev >= 0 && dev < kDev, DPK_ERR_ARG, "embed: device %d out of range", dev);
   const int variant = (C::RES2 ? 4 : 0) + (C::RES3 ? 2 : 0) + (C::IDT ? 1 : 0);
-  int& slots = cache[dev][fwd ? 0 : 1][variant][RESIDENT ? nnets : 0];
+  std::atomic<int>& kept = cache[dev][fwd ? 0 : 1][variant][RESIDENT ? nnets : 0];
+  int slots = kept.load(std::memory_order_relaxed);
   if (slots == 0) {
-    int ncu = 0, per_cu = 0;
-    DPK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    int per_cu = 0;
     if (fwd)
       DPK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fwd<E, RESIDENT, C>, 256, lds));
     else
       DPK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_bwd<E, RESIDENT, C>, 256, lds));
-    slots = (ncu < 1 ? 1 : ncu) * (per_cu < 1 ? 1 : per_cu);
+    slots = ncu * (per_cu < 1 ? 1 : per_cu);
+    kept.store(slots, std::memory_order_relaxed);
   }
   const int groups = cdiv(natoms, 4);
   const int pct = tune(DPK_TUNE_EMBED_GRID_PCT);

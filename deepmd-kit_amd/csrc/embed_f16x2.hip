@@ -36,6 +36,8 @@
 // 3.0e-7, 2.2e-5.
 // One wavefront an atom, or several where atoms are few (split_of), 16 slots a
 // tile; lane (g = lane / 16, c = lane % 16).
+#include <atomic>
+
 #include "dpk_common.h"
 #include "half16.h"
 #include "embed_image.h"
@@ -518,18 +520,18 @@ int launch2(bool fwd, void* out, const void* em, const void* gx, const int* atyp
             int d3, int natoms, int nnei, hipStream_t st) {
   // resident workgroups per device, cached per (device, direction, nnets, split)
   constexpr int kDev = 64, kRes = kResidentMaxBytes / NET_BYTES + 1;
-  static int cache[kDev][2][kRes][2];
+  static std::atomic<int> cache[kDev][2][kRes][2];
   int dev = 0, ncu = 0;
-  DPK_HIP(hipGetDevice(&dev));
+  const int rc = device_cus(&dev, &ncu);
+  if (rc != DPK_OK) return rc;
   DPK_REQUIRE(dev >= 0 && dev < kDev, DPK_ERR_ARG, "embed: device %d out of range", dev);
-  DPK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  if (ncu < 1) ncu = 1;
   const int lp = split_of(natoms, nnei, ncu);
   const bool bias4 = RESIDENT && fwd && nnets == 1;
   const size_t lds = (RESIDENT ? (size_t)nnets * NET_BYTES + (bias4 ? kBias4 : 0) : 0) +
                      (fwd && lp > 0 ? kPartSums : 0);
   const auto kfwd = bias4 ? k_fwd2<RESIDENT, RESIDENT, C> : k_fwd2<RESIDENT, false, C>;
-  int& slots = cache[dev][fwd ? 0 : 1][RESIDENT ? nnets : 0][lp > 0];
+  std::atomic<int>& kept = cache[dev][fwd ? 0 : 1][RESIDENT ? nnets : 0][lp > 0];
+  int slots = kept.load(std::memory_order_relaxed);
   if (slots == 0) {
     int per_cu = 0;
     if (fwd)
@@ -537,6 +539,7 @@ int launch2(bool fwd, void* out, const void* em, const void* gx, const int* atyp
     else
       DPK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_bwd2<RESIDENT, C>, 256, lds));
     slots = ncu * (per_cu < 1 ? 1 : per_cu);
+    kept.store(slots, std::memory_order_relaxed);
   }
   const int groups = cdiv(natoms, 4 >> lp);
   const int pct = tune(DPK_TUNE_EMBED_GRID_PCT);

@@ -698,12 +698,9 @@ int choose_split(const EmbArgs& A, int tiles, int ncu) {
 template <class SH>
 int launch64(bool fwd, EmbArgs& A, hipStream_t st) {
   constexpr int NW = kWaves;
-  static int ncu[64];
-  int dev = 0;
-  DPK_HIP(hipGetDevice(&dev));
-  DPK_REQUIRE(dev >= 0 && dev < 64, DPK_ERR_ARG, "embed: device %d out of range", dev);
-  if (ncu[dev] == 0)
-    DPK_HIP(hipDeviceGetAttribute(&ncu[dev], hipDeviceAttributeMultiprocessorCount, dev));
+  int dev = 0, ncu = 0;
+  const int rc = device_cus(&dev, &ncu);
+  if (rc != DPK_OK) return rc;
   constexpr int kMost = NW * (kFwdScratch<SH> > 4 * kGs<SH> ? kFwdScratch<SH> : 4 * kGs<SH>);
   constexpr int kRoom = (kLdsMax / 8 - kHead - kMost) / SH::size;
   static_assert(kRoom >= 1, "a net fits in LDS beside the scratch");
@@ -714,9 +711,9 @@ int launch64(bool fwd, EmbArgs& A, hipStream_t st) {
                         (size_t)A.room * SH::size);
   int tiles = 0;
   for (int t = 0; t < A.ntypes; ++t) tiles += (9 * (A.sec[t + 1] - A.sec[t]) / 10 + 15) / 16;
-  A.split = choose_split(A, tiles, ncu[dev]);
+  A.split = choose_split(A, tiles, ncu);
   const long want = ((long)A.natoms * A.split + NW - 1) / NW;
-  const unsigned grid = (unsigned)(want < ncu[dev] ? want : ncu[dev]);  // one workgroup a CU
+  const unsigned grid = (unsigned)(want < ncu ? want : ncu);  // one workgroup a CU
   const auto kernel = fwd ? (all ? k_fwd64<SH, true, NW> : k_fwd64<SH, false, NW>)
                           : (all ? k_bwd64<SH, true, NW> : k_bwd64<SH, false, NW>);
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * NW), lds, st, A);

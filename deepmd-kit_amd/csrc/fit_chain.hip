@@ -251,13 +251,8 @@ int run(int L, const int* w, const int* res, const void* const* params,
         const double* ebias, int nseg, const int* segs, double* atom_e, void* gxyz,
         const void* xyz, const int* order, int n, int d3, int m2, void* desc, void* ws,
         hipStream_t st) {
-  static int ncus[64];
-  int dev = 0;
-  DPK_HIP(hipGetDevice(&dev));
-  DPK_REQUIRE(dev >= 0 && dev < 64, DPK_ERR_ARG, "fit_chain: device %d out of range", dev);
-  if (ncus[dev] == 0)
-    DPK_HIP(hipDeviceGetAttribute(&ncus[dev], hipDeviceAttributeMultiprocessorCount, dev));
-  const int ncu = ncus[dev];
+  int dev = 0, ncu = 0, rc = device_cus(&dev, &ncu);
+  if (rc != DPK_OK) return rc;
   int hmax = 0;
   for (int l = 1; l <= L; ++l) hmax = w[l] > hmax ? w[l] : hmax;
   const size_t blk = (size_t)n * hmax;
@@ -265,7 +260,7 @@ int run(int L, const int* w, const int* res, const void* const* params,
   double* at = gd + (size_t)n * w[0];
   double *y[2] = {at, at + blk}, *gy[2] = {at + 2 * blk, at + 3 * blk},
     *gz[2] = {at + 4 * blk, at + 5 * blk}, *sd = at + 6 * blk;
-  int rc = dpk_fit_descriptor_fwd(desc, DPK_PREC_F64, xyz, order, n, d3, m2, st);
+  rc = dpk_fit_descriptor_fwd(desc, DPK_PREC_F64, xyz, order, n, d3, m2, st);
   if (rc != DPK_OK) return rc;
   // params of type t: four pointers a layer (W, W^T, b, idt), then w_out
   auto par = [&](int t, int l, int q) {

@@ -963,8 +963,8 @@ extern "C" int dpk_force_virial_cells(double* force, double* atom_virial, const 
   if (nw == 0) nw = natoms >= 96 * ncells ? 16 : (natoms >= 6 * ncells ? 8 : 4);
   nw = nw <= 4 ? 4 : (nw <= 8 ? 8 : 16);
   int dev = 0, ncu = 0;
-  DPK_HIP(hipGetDevice(&dev));
-  DPK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  const int rc = device_cus(&dev, &ncu);
+  if (rc != DPK_OK) return rc;
   // Workgroups a cell: three tables fit a CU's LDS, but a second and third
   // workgroup clears and adds a table of its own, so an ordinary cell has as many
   // as give half of that, and one of more than twice the mean (frames that differ)

@@ -726,11 +726,10 @@ int launch_search(const double* wrapped, const int* atype, const int* frame_of,
                   const int* cell_atoms, const int* img_pos, const double* shift_vec,
                   double rcut, const SelInfo& si, int natoms, int ncells, int* nlist,
                   int* status, bool ragged, hipStream_t st) {
-  int dev = 0, maxlds = 0;
-  DPK_HIP(hipGetDevice(&dev));
+  int dev = 0, ncu = 0, maxlds = 0;
+  const int rc = device_cus(&dev, &ncu);
+  if (rc != DPK_OK) return rc;
   DPK_HIP(hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-  int ncu = 0;
-  DPK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
   const size_t budget = (size_t)(maxlds < 160 * 1024 ? maxlds : 160 * 1024) - 512;
   const double per_cell = (double)natoms / ncells;
   int w = tune(DPK_TUNE_NLIST_WAVES);

@@ -42,6 +42,20 @@ int tune(int key) {
   return t ? t->v[key] : g_tune[key].load(std::memory_order_relaxed);
 }
 
+int device_cus(int* dev, int* ncu) {
+  constexpr int kDev = 64;
+  static std::atomic<int> cus[kDev];
+  DPK_HIP(hipGetDevice(dev));
+  const bool kept = *dev >= 0 && *dev < kDev;
+  *ncu = kept ? cus[*dev].load(std::memory_order_relaxed) : 0;
+  if (*ncu == 0) {
+    DPK_HIP(hipDeviceGetAttribute(ncu, hipDeviceAttributeMultiprocessorCount, *dev));
+    if (*ncu < 1) *ncu = 1;
+    if (kept) cus[*dev].store(*ncu, std::memory_order_relaxed);
+  }
+  return DPK_OK;
+}
+
 static int check_tune(const char* who, int key, int value) {
   if (key < 0 || key >= DPK_TUNE_COUNT) {
     set_error("%s: unknown key %d", who, key);

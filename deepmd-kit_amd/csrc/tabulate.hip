@@ -15,8 +15,6 @@
 // forward and grad_grad put the L channels on the threads and walk the
 // neighbours, grad puts the neighbours on the threads and walks the channels,
 // with dy for the atom staged in LDS.
-#include <atomic>
-
 #include "dpk_common.h"
 
 namespace dpk {
@@ -612,14 +610,9 @@ int launch_tab4(bool fwd, Tab4<T>& A, hipStream_t st) {
   }
   A.lp = 0;
   if (!fwd) {
-    static std::atomic<int> ncus[64];  // CUs of a device, asked for once
-    int dev = 0;
-    DPK_HIP(hipGetDevice(&dev));
-    int ncu = dev >= 0 && dev < 64 ? ncus[dev].load(std::memory_order_relaxed) : 0;
-    if (ncu == 0) {
-      DPK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-      if (dev >= 0 && dev < 64) ncus[dev].store(ncu, std::memory_order_relaxed);
-    }
+    int dev = 0, ncu = 0;
+    const int rc = device_cus(&dev, &ncu);
+    if (rc != DPK_OK) return rc;
     A.lp = tab_split(A.natoms, A.nnei, ncu);
   }
   const dim3 g(cdiv((long long)A.natoms << A.lp, 4));
