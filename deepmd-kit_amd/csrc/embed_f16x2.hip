@@ -19,14 +19,14 @@
 //    and lo parts share one 16x16x32 instruction;
 //  * the backward adds up the gx of the two channels that carry one resnet
 //    copy once an atom.
-// Measured against tanh itself, all of G re-laid and every copy contracted:
-// 131,072 Cu atoms (12 tiles an atom) forward 2.47 -> 2.30 ms, backward 3.79 ->
-// 3.64; three wavefronts a SIMD for the backward without its 32 bytes of
-// scratch (outside the loop) 3.74, five for the forward 2.32 (all at one
-// workgroup per resident slot; kGridRounds takes the two to 1.79 and 2.96).
+// Measured in one run, against all of G re-laid, every copy contracted and one
+// workgroup per resident slot: 131,072 Cu atoms (12 tiles an atom) forward 2.26 ->
+// 1.94 ms, backward 3.57 -> 3.10 (under the profiler 1.99 and 3.16).  Three
+// wavefronts a SIMD for the backward and five for the forward gain nothing.
 //
 // Precision.  The split operands are tanh, not r (whose 1/2 would cancel in the
-// sums; 32 FMAs a tile, 131,072 Cu atoms 7.77 -> 7.97 ms a step), and tangents
+// sums; 32 FMAs a tile: forward 1.88 -> 1.94 ms, backward 3.05 -> 3.10, a step of
+// 131,072 Cu atoms 7.68 -> 7.78), and tangents
 // at one to two times their value (layers12); the resnet copies have an
 // accumulator of their own.  Errors against 64 bits, 2-norms, weights exact in
 // FP16 and scaled by 1 / 0.3 / 0.1 (nets of 32, 64, 128), r and quarter-scale
@@ -496,7 +496,8 @@ constexpr int kPartSums = 4 * 8 * 16 * 16;  // forward, split atoms: four wavefr
 // Workgroups of a persistent grid per resident slot: with one, a slow XCD or a
 // ragged last round holds the launch; with eight, finished slots take what is
 // left, and a net is still copied to LDS once for several groups of atoms.
-// Forward + backward us with 1 / 4 / 8 a slot, or one a group: Cu (one net)
+// Forward + backward us (before tanh took r's place: 1-2% less than now) with 1 /
+// 4 / 8 a slot, or one a group: Cu (one net)
 // 8,788 atoms 356 / 333 / 331 / 332, 20,000 782 / 705 / 704 / 705, 131,072 5,227 /
 // 4,703 / 4,748 / 4,658; water (two nets) 8,788 275 / 275 / 276 / 274, 49,000 1,468 /
 // 1,418 / 1,399 / 1,435, 131,072 3,974 / 3,828 / 3,792 / 3,917.
