@@ -140,6 +140,7 @@ def test_embed_f64_nan_and_infinity():
     ([32, 64, 128], [33, 18], True, 1100, {}),        # all atoms in both groups, whole and split
     ([32, 64, 128], [33, 18], True, 300, {}),
     ([32, 64, 128], [2, 3], False, 16500, {}),        # more than 64 atoms a workgroup
+    ([10, 20, 40], [2] * 16, False, 90, {}),          # 256 nets, the most there can be
     ([20, 30, 100], [30, 20], False, 700, {"dt": True}),
     ([25, 50, 100], [30, 20], False, 600, {"act": "gelu"}),
 ])
