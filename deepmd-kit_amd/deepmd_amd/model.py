@@ -510,8 +510,9 @@ class Fitting:
         return (len(flat) == 1 and 128 < min(flat) <= 256 and len({len(w) for w in hs}) == 1
                 and len(hs[0]) in (2, 3))
 
-    def buffers(self, n: int):
-        """Per-system work buffers for n slots (flat; viewed per layer)."""
+    def buffers(self, n: int, segments=None):
+        """Per-system work buffers for n slots (flat; viewed per layer).
+        ``segments`` as in run() (default: slots of every type)."""
         dev, rd, gd = self.device, self.real_dtype, self.gemm_dtype
         hmax = max(self.widths)
         nl = len(self.widths)
@@ -522,7 +523,9 @@ class Fitting:
                     "D": torch.empty((nd, 2 * self.din), dtype=gd, device=dev),
                     "GD": torch.empty((nd, self.din), dtype=torch.float32, device=dev),
                     "cx": None}
-        if self.chain is not None and n <= len(self.nets) * self.chain_rows(hmax):
+        # types without a slot add no rows and no launches
+        types = len(self.nets) if segments is None else sum(b > a for _, a, b in segments)
+        if self.chain is not None and n <= max(types, 1) * self.chain_rows(hmax):
             nb = int(lib().dpk_fit_chain_f64_workspace_bytes(n, nl, self.chain["widths"][1]))
             return {"D": torch.empty((n, self.din), dtype=gd, device=dev),
                     "ws": torch.empty(max(nb, 1), dtype=torch.uint8, device=dev)}
@@ -1016,7 +1019,7 @@ class SeAModel:
         sysd.desc = torch.empty((N, self.d3 * self.axis_neuron), dtype=ddt, device=dev)
         sysd.gxyz = torch.empty((N, 4, self.d3), dtype=real, device=dev)
         sysd.atom_e = torch.empty(N, dtype=torch.float64, device=dev)
-        sysd.fit = self.fitting.buffers(sysd.nreal)
+        sysd.fit = self.fitting.buffers(sysd.nreal, segments)
         sysd.nd = torch.empty((N, S, 4), dtype=real, device=dev)
         sysd.force = torch.empty((N, 3), dtype=torch.float64, device=dev)
         sysd.vrow = torch.empty(int(lib.dpk_force_virial_workspace_bytes(N)), dtype=torch.uint8,
@@ -1189,7 +1192,7 @@ class SeAModel:
                 order, s.segments = self._slot_order(at.cpu().numpy())
                 s.order[:order.size].copy_(torch.from_numpy(order))
                 s.nreal = int(order.size)
-                s.fit = self.fitting.buffers(max(s.nreal, 1))
+                s.fit = self.fitting.buffers(max(s.nreal, 1), s.segments)
                 s.extra["types_key"] = key
             if self.nx:
                 self.set_params(s, fparam, aparam)

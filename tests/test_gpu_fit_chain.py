@@ -101,3 +101,29 @@ def test_fit_chain_not_finite(rows, bad):
     for a, b in zip(*out):
         assert np.array_equal(a[keep], b[keep])
     assert not np.isfinite(out[1][1][at]).all()
+
+
+def test_fit_chain_rows_of_present_types():
+    """The form is chosen by the rows of the types that have slots, not by the
+    number of nets; both forms give the same energies there."""
+    rng = np.random.default_rng(7)
+    h, d3, m2, nx = 512, 8, 4, M.Fitting.chain_rows(512)
+    n = int(nx) + 40
+    nets = [M._layers(M._rand_net(rng, [d3 * m2, h, h, 1], True, True)) for _ in range(2)]
+    fit = M.Fitting(nets, np.zeros(2), np.zeros(2), "f64", torch.device(DEV))
+    one, two = [(0, 0, n), (1, n, n)], [(0, 0, n // 2), (1, n // 2, n)]
+    assert "ws" not in fit.buffers(n, one)
+    assert "ws" in fit.buffers(n, two) and "ws" in fit.buffers(n)
+    assert "ws" in fit.buffers(n - 40, one) and "ws" in fit.buffers(1, [(0, 0, 0), (1, 0, 0)])
+    order = torch.arange(n, dtype=torch.int32, device=DEV)
+    xyz = torch.tensor(rng.normal(size=(n, 4, d3)) * 0.3, device=DEV)
+    out = []
+    for bf in (fit.buffers(n, one), fit.buffers(n)):
+        ae = torch.zeros(n, dtype=torch.float64, device=DEV)
+        gx = torch.zeros((n, 4, d3), dtype=torch.float64, device=DEV)
+        fit.run(ae, gx, xyz, order, one, n, bf, d3, m2, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        out.append((ae.cpu().numpy(), gx.cpu().numpy()))
+    for a, b in zip(*out):
+        # sums of at most 512 FP64 products a layer, four layers' depth
+        assert np.abs(a - b).max() <= 512 * 4 * 2.3e-16 * max(np.abs(b).max(), 1.0)
